@@ -48,6 +48,10 @@ ek::Res to_res(const echokv_residual* r) {
   return d;
 }
 
+// Page of chunk id = umulhi(id, chunk_mul(KC)), 0: the id itself. ceil(2^32 / KC) is exact
+// for ids < 2^24 and KC <= 4 (fractions of id / KC are multiples of 1 / KC >= 1/4).
+uint32_t chunk_mul(int KC) { return KC == 1 ? 0u : (uint32_t)((0x100000000ull + KC - 1) / KC); }
+
 int launched(hipError_t e) { return e == hipSuccess ? ECHOKV_OK : ECHOKV_ELAUNCH; }
 
 }  // namespace
@@ -252,10 +256,7 @@ int decode_run(const echokv_layout* L, const uint8_t* pages, const int64_t* bloc
   a.bs_shift = mfma ? __builtin_ctz((unsigned)L->block_size) : 0;
   a.kg_shift = mfma ? __builtin_ctz((unsigned)L->k_group) : 0;
   a.vg_shift = __builtin_ctz((unsigned)L->v_group);
-  // ceil(2^32 / KC) is exact for chunk ids < 2^24 (fractions of id / KC are multiples of 1 / KC >= 1/4).
-  a.kc_mul = !mfma || L->chunks_per_page == 1
-                 ? 0u
-                 : (uint32_t)((0x100000000ull + L->chunks_per_page - 1) / L->chunks_per_page);
+  a.kc_mul = mfma ? chunk_mul(L->chunks_per_page) : 0u;
   if (!mfma && num_seqs > INT32_MAX / L->num_kv_heads / num_splits) return ECHOKV_ESHAPE;  // one workgroup each
   if (static_scratch) {
     // acc [S, Hq, splits, D] then ml [S, Hq, splits, 2], float32, in the static array.
@@ -364,11 +365,15 @@ int64_t echokv_decode_workspace_rows(const echokv_layout* L, int32_t num_q_heads
   return rows < split_rows ? rows : split_rows;
 }
 
-int echokv_prefill(const echokv_layout* L, const uint8_t* pages, const int64_t* block_res, const int64_t* res_group,
-                   const echokv_residual* res, const void* query, int64_t q_s0, int64_t q_s1, int32_t q_dtype,
-                   int32_t num_q_heads, void* out, int64_t o_s0, int64_t o_s1, int32_t out_dtype,
-                   const int32_t* tiles, int64_t n_tiles, int32_t tile_m, const int32_t* block_table, int64_t bt_s0,
-                   float softmax_scale, int32_t own_group, float* lse, echokv_stream_t stream) {
+namespace {
+
+// echokv_prefill and echokv_prefill_split: the checks, then the kernels.
+int prefill_run(const echokv_layout* L, const uint8_t* pages, const int64_t* block_res, const int64_t* res_group,
+                const echokv_residual* res, const void* query, int64_t q_s0, int64_t q_s1, int32_t q_dtype,
+                int32_t num_q_heads, void* out, int64_t o_s0, int64_t o_s1, int32_t out_dtype,
+                const int32_t* tiles, int64_t n_tiles, int32_t tile_m, const int32_t* block_table, int64_t bt_s0,
+                float softmax_scale, int32_t own_group, float* lse, int32_t n_splits, int32_t split_keys,
+                int64_t part_rows, float* acc, float* ml, echokv_stream_t stream) {
   if (!lay_ok(L)) return ECHOKV_ESHAPE;
   if (num_q_heads <= 0 || num_q_heads % L->num_kv_heads) return ECHOKV_ESHAPE;
   const int gqa = num_q_heads / L->num_kv_heads;
@@ -382,6 +387,8 @@ int echokv_prefill(const echokv_layout* L, const uint8_t* pages, const int64_t* 
   if (own_group && (L->k_group & (L->k_group - 1))) return ECHOKV_ESHAPE;
   if (!dtype_ok(q_dtype) || !dtype_ok(out_dtype)) return ECHOKV_EDTYPE;
   if (n_tiles < 0 || !res_ok(res)) return ECHOKV_EINVAL;
+  if (n_splits < 1 || n_splits > ek::kPrefillMaxSplits || split_keys < 1 || split_keys % 128) return ECHOKV_EINVAL;
+  if (n_splits > 1 && (!mfma || !acc || !ml || part_rows < 1)) return ECHOKV_EINVAL;
   if (n_tiles == 0) return ECHOKV_OK;
   if (!pages || !block_res || !res_group || !query || !out || !tiles || !block_table) return ECHOKV_EINVAL;
   ek::PrefillArgs a;
@@ -408,6 +415,21 @@ int echokv_prefill(const echokv_layout* L, const uint8_t* pages, const int64_t* 
   a.lse = lse;
   a.g0 = 0;
   a.gs = gqa;
+  a.n_splits = n_splits;
+  a.split_keys = split_keys;
+  a.part_rows = part_rows;
+  a.acc = acc;
+  a.ml = ml;
+  const int KC = L->chunks_per_page;
+  a.bs_shift = __builtin_ctz((unsigned)L->block_size);
+  a.kg_shift = __builtin_ctz((unsigned)L->k_group);
+  a.kc_mul = chunk_mul(KC);
+  const int qa = q_dtype == ECHOKV_F32 ? 4 : 8;  // elements per 16 bytes
+  const uintptr_t oa = out_dtype == ECHOKV_F32 ? 16 : 8;
+  a.fast = !(L->block_size & (L->block_size - 1)) && !(L->k_group & (L->k_group - 1)) && L->k_group >= 4 &&
+           L->v_group % 8 == 0 && KC <= 4 && L->num_blocks * KC < (1LL << 24) && (uintptr_t)pages % 16 == 0 &&
+           (uintptr_t)query % 16 == 0 && q_s0 % qa == 0 && q_s1 % qa == 0 && (uintptr_t)out % oa == 0 &&
+           o_s0 % 4 == 0 && o_s1 % 4 == 0;
   if (mfma) return launched(ek::launch_prefill(a, n_tiles, (hipStream_t)stream));
   if (n_tiles > INT32_MAX / L->num_kv_heads) return ECHOKV_EINVAL;
   for (int g0 = 0; g0 < gqa; g0 += 16) {  // passes of 16 query heads per KV head
@@ -416,6 +438,30 @@ int echokv_prefill(const echokv_layout* L, const uint8_t* pages, const int64_t* 
     if (ek::launch_prefill_any(a, n_tiles, (hipStream_t)stream) != hipSuccess) return ECHOKV_ELAUNCH;
   }
   return ECHOKV_OK;
+}
+
+}  // namespace
+
+int echokv_prefill(const echokv_layout* L, const uint8_t* pages, const int64_t* block_res, const int64_t* res_group,
+                   const echokv_residual* res, const void* query, int64_t q_s0, int64_t q_s1, int32_t q_dtype,
+                   int32_t num_q_heads, void* out, int64_t o_s0, int64_t o_s1, int32_t out_dtype,
+                   const int32_t* tiles, int64_t n_tiles, int32_t tile_m, const int32_t* block_table, int64_t bt_s0,
+                   float softmax_scale, int32_t own_group, float* lse, echokv_stream_t stream) {
+  return prefill_run(L, pages, block_res, res_group, res, query, q_s0, q_s1, q_dtype, num_q_heads, out, o_s0, o_s1,
+                     out_dtype, tiles, n_tiles, tile_m, block_table, bt_s0, softmax_scale, own_group, lse, 1, 128, 0,
+                     nullptr, nullptr, stream);
+}
+
+int echokv_prefill_split(const echokv_layout* L, const uint8_t* pages, const int64_t* block_res,
+                         const int64_t* res_group, const echokv_residual* res, const void* query, int64_t q_s0,
+                         int64_t q_s1, int32_t q_dtype, int32_t num_q_heads, void* out, int64_t o_s0, int64_t o_s1,
+                         int32_t out_dtype, const int32_t* tiles, int64_t n_tiles, int32_t tile_m,
+                         const int32_t* block_table, int64_t bt_s0, float softmax_scale, int32_t own_group, float* lse,
+                         int32_t n_splits, int32_t split_keys, int64_t part_rows, float* acc, float* ml,
+                         echokv_stream_t stream) {
+  return prefill_run(L, pages, block_res, res_group, res, query, q_s0, q_s1, q_dtype, num_q_heads, out, o_s0, o_s1,
+                     out_dtype, tiles, n_tiles, tile_m, block_table, bt_s0, softmax_scale, own_group, lse, n_splits,
+                     split_keys, part_rows, acc, ml, stream);
 }
 
 int64_t echokv_prefill_dense_workspace(const echokv_layout* L, int64_t n_packs) {

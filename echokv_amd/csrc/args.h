@@ -251,7 +251,22 @@ struct PrefillArgs {
   int og_mask;  // nonzero: a query at position p sees keys < (p & og_mask) (its own K group left out)
   float* lse;   // nullable: [rows, hq] log2-domain log-sum-exp of each query row's scores
   int g0, gs;   // fp32 kernel (prefill_any): this pass's query heads of each KV head, gs <= 16
+  // MFMA kernel: a tile's context in ranges of split_keys keys (a multiple of 128), at
+  // most n_splits of them (the last takes the rest). With n_splits > 1, range z of query
+  // row r and head qh leaves its unnormalized output and (max in log2 units, sum) in row
+  // (z * part_rows + r) * hq + qh of acc [.., D] and ml [.., 2].
+  int n_splits, split_keys;
+  long part_rows;
+  float* acc;
+  float* ml;
+  // 1: the MFMA kernel's items (4 keys x 8 channels) sit in one K group and V group, the
+  // block size and K group are powers of two (bs_shift, kg_shift: their logs), chunk ids
+  // are under 2^24 (page = umulhi(id, kc_mul); kc_mul 0: one chunk a page), and query /
+  // output rows are aligned for 16-byte loads / four-channel stores.
+  int fast, bs_shift, kg_shift;
+  uint32_t kc_mul;
 };
+constexpr int kPrefillMaxSplits = 64;
 
 struct PackArgs {
   Lay L;

@@ -533,6 +533,57 @@ def test_head_size_256_prefill_on_the_mfma_kernel(device, h, gqa, dt, bits):
     check(f"prefill D256 H{h} GQA{gqa} {str(dt)[6:]} int{bits}", out, ref)
 
 
+@pytest.mark.parametrize("d,gqa,bs,kg,vg,dt,og", [
+    (128, 4, 16, 16, 32, torch.float16, False),
+    (128, 4, 64, 32, 32, torch.bfloat16, True),   # own-group part: the ranges' log-sum-exp
+    (64, 7, 128, 64, 32, torch.float32, False),   # query lo part
+    (256, 4, 32, 32, 32, torch.bfloat16, False),
+    (128, 1, 48, 16, 64, torch.float16, False),   # items read element by element: block size,
+    (64, 4, 16, 16, 4, torch.float16, False)])    # V group
+def test_fused_prefill_key_ranges_at_their_edges(device, monkeypatch, d, gqa, bs, kg, vg, dt, og):
+    """The fused kernel's key ranges (128 keys here): contexts on and around the range
+    boundaries, chunks crossing them, one-range tiles beside many-range ones, the
+    range-count cap (a last range that takes the rest), a negative softmax scale and
+    query rows that are not 16-byte aligned; against the oracle."""
+    monkeypatch.setattr(pf, "SPLIT_MIN_KEYS", 128)
+    monkeypatch.setattr(pf, "SPLIT_SLOTS", 1 << 20)
+    lens = np.array([1, 127, 128, 129, 255, 257, 300, 1000])
+    h = 2
+    store, table = build_layer(device, lens, 4, h=h, d=d, bs=bs, kg=kg, vg=vg, dtype=dt, seed=31)
+    ps = oracle_view(store)
+    table_d = torch.from_numpy(table).to(device, torch.int32)
+    prefill, row = [], 0
+    for i, n in enumerate(lens.tolist()):
+        nq = min(n, (1, 40, 64, 5, 17, 64, 33, 64)[i])
+        prefill.append((row, row + nq, n, 0))
+        row += nq
+    reqs = list(range(len(lens)))
+    gen = torch.Generator(device=device)
+    gen.manual_seed(310)
+    wide = torch.randn(row, gqa * h, d + 3, device=device, generator=gen).to(dt)
+    for scale, q, cap in ((d ** -0.5, wide[..., :d].contiguous(), 64), (-0.05, wide[..., 3:], 64),
+                          (d ** -0.5, wide[..., :d].contiguous(), 3)):
+        if og and scale < 0:
+            continue  # the own-group part alone takes any scale; its first part is what is tested here
+        monkeypatch.setattr(pf, "SPLIT_MAX", 64)
+        assert pf.fused_splits(prefill, pf.block_m(gqa, d), h) == (8, 128)
+        if cap == 3:  # fewer ranges than the contexts need
+            monkeypatch.setattr(pf, "fused_splits", lambda *_: (3, 128))
+        out = torch.zeros(row, gqa * h, d, device=device)
+        kw = {}
+        if og:
+            key = torch.randn(row, h, d, device=device, generator=gen).to(dt)
+            kw = {"own_group_key": key}
+        pf.prefill_attention(store, q, out, prefill, reqs, table_d, scale, **kw)
+        torch.cuda.synchronize()
+        qn = q.float().cpu().numpy()
+        if og:
+            ref = OA.prefill_own_group_exact(ps, qn, key.float().cpu().numpy(), prefill, reqs, table, scale)
+        else:
+            ref = OA.prefill_attention(ps, qn, prefill, reqs, table, scale, vectorized=True)
+        check(f"prefill ranges D{d} GQA{gqa} bs{bs} kg{kg} vg{vg} {str(dt)[6:]} scale {scale:.3f} cap {cap}", out, ref)
+
+
 @pytest.mark.parametrize("bits", [2, 4, 8])
 def test_decode_over_a_layer_view_spanning_more_than_4_gib(device, bits):
     """One layer's view of a pool interleaved across 32 layers (page stride = 32
