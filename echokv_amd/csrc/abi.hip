@@ -253,11 +253,15 @@ int decode_run(const echokv_layout* L, const uint8_t* pages, const int64_t* bloc
   a.tier = tier;
   a.tier0 = tier;
   a.tier_mask = nullptr;
-  a.bs_shift = mfma ? __builtin_ctz((unsigned)L->block_size) : 0;
-  a.kg_shift = mfma ? __builtin_ctz((unsigned)L->k_group) : 0;
+  a.bs_shift = __builtin_ctz((unsigned)L->block_size);
+  a.kg_shift = __builtin_ctz((unsigned)L->k_group);
   a.vg_shift = __builtin_ctz((unsigned)L->v_group);
-  a.kc_mul = mfma ? chunk_mul(L->chunks_per_page) : 0u;
-  if (!mfma && num_seqs > INT32_MAX / L->num_kv_heads / num_splits) return ECHOKV_ESHAPE;  // one workgroup each
+  a.kc_mul = chunk_mul(L->chunks_per_page);
+  a.any_fast = !(L->block_size & (L->block_size - 1)) && !(L->k_group & (L->k_group - 1)) && L->k_group >= 4 &&
+               L->v_group % 8 == 0 && L->head_size % 8 == 0 && L->num_kv_heads * L->head_size % 32 == 0 &&
+               L->chunks_per_page <= 4 && L->num_blocks * L->chunks_per_page < (1LL << 24) &&
+               (uintptr_t)pages % 16 == 0;
+  if (!mfma && num_seqs > INT32_MAX / L->num_kv_heads / num_splits) return ECHOKV_ESHAPE;  // grid x
   if (static_scratch) {
     // acc [S, Hq, splits, D] then ml [S, Hq, splits, 2], float32, in the static array.
     if (num_seqs > (1LL << 31) / num_q_heads / num_splits) return ECHOKV_ETOOBIG;

@@ -197,6 +197,9 @@ struct DecodeArgs {
   // chunk id / chunks_per_page: floor(id / KC) = umulhi(id, kc_mul) (kc_mul 0: KC = 1).
   int bs_shift, kg_shift, vg_shift;
   uint32_t kc_mul;
+  // decode_any: 1 if its items (4 keys x 8 channels) sit in one K group and V group, block
+  // size and K group are powers of two, chunk ids fit kc_mul and rows are 8-byte aligned.
+  int any_fast;
   float* acc;  // [S, Hq, splits, D]
   float* ml;   // [S, Hq, splits, 2] = (running max in log2 units, sum)
   // Balanced schedule (ranges > 0): `ranges` equal block ranges; partial slot p of

@@ -42,13 +42,12 @@
 // A split covers max(blocks_per_split, ceil(blocks / num_splits)) blocks of
 // the sequence's own length, so results do not depend on the rest of the
 // batch; a second kernel merges the splits in order (log-sum-exp, log2 units).
-#include "args.h"
+#include "items.h"
 
 namespace ek {
 
 typedef uint32_t u4_t __attribute__((ext_vector_type(4)));
 
-__device__ __forceinline__ h2_t u2h(uint32_t u) { return __builtin_bit_cast(h2_t, u); }
 __device__ __forceinline__ uint32_t h2u(h2_t h) { return __builtin_bit_cast(uint32_t, h); }
 __device__ __forceinline__ h8_t w2h8(uint32_t a, uint32_t b, uint32_t c, uint32_t d) {
   return __builtin_bit_cast(h8_t, u4_t{a, b, c, d});

@@ -32,13 +32,11 @@
 // header and step i + 3's table entry are requested before step i's products.
 // Items whose keys or channels straddle a group (K group not a multiple of 4, V
 // group not of 8) are read element by element instead.
-#include "args.h"
+#include "items.h"
 
 namespace ek {
 
 namespace {
-
-__device__ __forceinline__ h2_t u2h_(uint32_t u) { return __builtin_bit_cast(h2_t, u); }
 
 // max / sum over lanes l, l ^ 16, l ^ 32, l ^ 48 (every lane gets the result).
 __device__ __forceinline__ float rows_max(float x) {
@@ -67,39 +65,6 @@ struct Raw {
   int rg;                 // K group of the block's residual slot (if it has one)
   bool ok;                // the item's keys can be read
 };
-
-// Eight codes, `sh` bits into the 8 bytes w, as fp16 pairs (exact). A byte b < 16 read as
-// E4M3 is b * 2^-9, so the fp8 conversion with scale 2^9 gives INT4 / INT2 codes; INT8
-// codes take the exponent of 1024.
-template <int BITS>
-__device__ __forceinline__ void code_pairs(uint2 w, int sh, h2_t c[4]) {
-  if constexpr (BITS == 8) {
-    const uint32_t m = 0x64646464u;
-    const h2_t k = {(_Float16)1024.0f, (_Float16)1024.0f};
-    c[0] = u2h_(__builtin_amdgcn_perm(m, w.x, 0x04010400u)) - k;
-    c[1] = u2h_(__builtin_amdgcn_perm(m, w.x, 0x04030402u)) - k;
-    c[2] = u2h_(__builtin_amdgcn_perm(m, w.y, 0x04010400u)) - k;
-    c[3] = u2h_(__builtin_amdgcn_perm(m, w.y, 0x04030402u)) - k;
-  } else {
-    const uint32_t x = (uint32_t)(((uint64_t)w.y << 32 | w.x) >> sh);
-    uint32_t a, b;  // channels 0..3, 4..7, a byte each
-    if constexpr (BITS == 4) {
-      const uint32_t lo = x & 0x0f0f0f0fu, hi = (x >> 4) & 0x0f0f0f0fu;  // even / odd channels
-      a = __builtin_amdgcn_perm(hi, lo, 0x05010400u);
-      b = __builtin_amdgcn_perm(hi, lo, 0x07030602u);
-    } else {
-      const uint32_t y0 = x & 0x03030303u, y1 = (x >> 2) & 0x03030303u;  // byte b of y_k: channel 4b + k
-      const uint32_t y2 = (x >> 4) & 0x03030303u, y3 = (x >> 6) & 0x03030303u;
-      const uint32_t p = __builtin_amdgcn_perm(y1, y0, 0x05010400u), q = __builtin_amdgcn_perm(y3, y2, 0x05010400u);
-      a = __builtin_amdgcn_perm(q, p, 0x05040100u);
-      b = __builtin_amdgcn_perm(q, p, 0x07060302u);
-    }
-    c[0] = __builtin_amdgcn_cvt_scalef32_pk_f16_fp8(a, 512.0f, false);
-    c[1] = __builtin_amdgcn_cvt_scalef32_pk_f16_fp8(a, 512.0f, true);
-    c[2] = __builtin_amdgcn_cvt_scalef32_pk_f16_fp8(b, 512.0f, false);
-    c[3] = __builtin_amdgcn_cvt_scalef32_pk_f16_fp8(b, 512.0f, true);
-  }
-}
 
 // Four consecutive elements by one store (aligned). DT is a template parameter so that
 // the dtype branch sits outside the caller's loop (the kernel's code is fetched cold
@@ -259,10 +224,10 @@ __global__ __launch_bounds__(256, QLO && D > 64 ? 1 : 2) void prefill_kernel(Pre
           float x8[8];
 #pragma unroll
           for (int e = 0; e < 8; ++e)
-            x8[e] = __builtin_fmaf((float)c[e >> 1][e & 1], (float)u2h_(sw[e >> 1])[e & 1], (float)u2h_(mw[e >> 1])[e & 1]);
+            x8[e] = __builtin_fmaf((float)c[e >> 1][e & 1], (float)u2h(sw[e >> 1])[e & 1], (float)u2h(mw[e >> 1])[e & 1]);
           put_k(i, x8);
           code_pairs<B>(w.v[i], sh, c);
-          const h2_t vs = u2h_(w.vs[i] * 0x10001u), vm = u2h_(w.vm[i] * 0x10001u);
+          const h2_t vs = u2h(w.vs[i] * 0x10001u), vm = u2h(w.vm[i] * 0x10001u);
 #pragma unroll
           for (int e = 0; e < 4; ++e) v[i][e] = __builtin_elementwise_fma(c[e], vs, vm);
           __builtin_amdgcn_sched_barrier(0);

@@ -473,6 +473,34 @@ def test_layouts_outside_the_mfma_kernels(device, d, bs, kg, vg, h, gqa, bits):
     check(f"prefill {label}", out, ref)
 
 
+@pytest.mark.parametrize("d,bs,kg,vg,h,gqa,dt", [
+    (48, 16, 16, 16, 2, 4, torch.bfloat16),   # rows of 8 lanes
+    (64, 32, 8, 32, 3, 7, torch.float32),     # two workgroups of query heads
+    (96, 64, 32, 24, 4, 1, torch.float16),    # one query head
+    (160, 16, 16, 32, 2, 3, torch.bfloat16),  # two items a lane, the second ones partly past the head
+    (36, 16, 16, 12, 2, 5, torch.float32),    # half an octet: element by element
+    (128, 32, 4, 64, 2, 4, torch.float16)])   # a K group is one item
+@pytest.mark.parametrize("bits", [8, 4, 2])
+def test_fp32_decode_items_at_their_edges(device, d, bs, kg, vg, h, gqa, dt, bits):
+    """The fp32 decode kernel's items (4 keys x 8 channels): contexts ending inside, on and
+    past an item, a batch and a split, open K groups in the residual's dtype, splits of
+    one block and more splits than a sequence has; against the oracle. The kernel
+    computes in fp32: weights carry the scores' rounding, about 2^-24 x |score| in log2
+    units (|score| < 100 here), and outputs are sums of values up to 40."""
+    lens = np.array([1, 3, 4, 5, 15, 16, 17, 33, 63, 65, 130, 257])
+    store, table = build_layer(device, lens, bits, h=h, d=d, bs=bs, kg=kg, vg=vg, dtype=dt, seed=9, outliers=0.02)
+    ps = oracle_view(store)
+    gen = torch.Generator(device=device)
+    gen.manual_seed(90)
+    q = torch.randn(len(lens), gqa * h, d, device=device, generator=gen).to(dt)
+    ref = OA.decode_attention(ps, q.float().cpu().numpy(), table, lens, d ** -0.5, vectorized=True)
+    for bps, ns in ((1, 40), (2, 3), (16, 32)):
+        got = dec.decode_attention(store, q, torch.from_numpy(table).to(device, torch.int32),
+                                   torch.from_numpy(lens).to(device), d ** -0.5, blocks_per_split=bps, num_splits=ns)
+        torch.cuda.synchronize()
+        check(f"fp32 decode D{d} kg{kg} vg{vg} GQA{gqa} int{bits} bps{bps}", got, ref, tol=4e-4)
+
+
 @pytest.mark.parametrize("h,gqa,vg,dt", [(8, 4, 32, torch.float16), (3, 4, 64, torch.bfloat16), (1, 20, 16, torch.float32),
                                          (2, 8, 128, torch.float16)])
 @pytest.mark.parametrize("bits", [8, 4, 2])
