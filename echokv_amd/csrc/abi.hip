@@ -602,12 +602,17 @@ int echokv_canary_kl(const void* query, int32_t q_dtype, int64_t q_sl, int64_t q
   }
   // Only the last floor(window / k_group) * k_group keys are scored.
   if (head_size < 1 || head_size > ek::kCanaryMaxD || window < k_group) return ECHOKV_ESHAPE;
-  const int rows = (num_q_heads / num_kv_heads) * nq;  // query rows one workgroup scores
-  if (ek::canary_lds_bytes(head_size, nbits, rows) > ek::kLdsBytes) return ECHOKV_ESHAPE;
+  if (ek::canary_lds_bytes(head_size, nbits, k_group) > ek::kLdsBytes) return ECHOKV_ESHAPE;
+  // Query rows per KV head: what four variants' keys beside the rows' state leave in a CU's
+  // LDS (the kernel itself takes the rows 64 at a time).
+  const int64_t rows = (int64_t)(num_q_heads / num_kv_heads) * nq, variants = 1 + nbits, keys = head_size <= 128 ? 64 : 32;
+  if (4 * (variants * keys * (head_size + 1) + 2 * keys + 4 + variants * rows * 2 + rows) > (int64_t)ek::kLdsBytes)
+    return ECHOKV_ESHAPE;
   if (num_layers == 0) return ECHOKV_OK;
   if (!query || !kref || !partial || !out) return ECHOKV_EINVAL;
+  const int k_vec = head_size % 4 == 0 && (uintptr_t)kref % 16 == 0 && k_sl % 4 == 0 && k_s0 % 4 == 0 && k_s1 % 4 == 0;
   ek::CanaryArgs a{query, q_dtype, q_sl, q_s0, q_s1, kref, k_sl, k_s0, k_s1, nq, num_q_heads, num_kv_heads,
-                   head_size, window, nbits, bits_packed, k_group, softmax_scale, partial, out};
+                   head_size, window, nbits, bits_packed, k_group, softmax_scale, k_vec, partial, out};
   return launched(ek::launch_canary(a, num_layers, (hipStream_t)stream));
 }
 

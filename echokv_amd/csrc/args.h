@@ -231,6 +231,7 @@ struct CanaryArgs {
   long k_sl, k_s0, k_s1;
   int nq, hq, h, d, window, nbits, bits_packed, kg;
   float scale;
+  int k_vec;  // 1: every key row is aligned for 16-byte loads and whole in them
   float* partial;  // [layers, H, nbits]: KL sums of each (layer, KV head)
   float* out;
 };
@@ -345,7 +346,7 @@ hipError_t launch_merge_any(const MergeArgs& a, hipStream_t s);
 inline int any_tile_tokens(int gqa) { return gqa >= 16 ? 1 : 16 / gqa; }
 hipError_t launch_prefill_any(const PrefillArgs& a, long n_tiles, hipStream_t s);
 hipError_t launch_canary(const CanaryArgs& a, int num_layers, hipStream_t s);
-size_t canary_lds_bytes(int d, int nbits, int rows);  // one canary workgroup's LDS
+size_t canary_lds_bytes(int d, int nbits, int kg);  // one canary workgroup's LDS
 hipError_t launch_prefill(const PrefillArgs& a, long n_tiles, hipStream_t s);
 hipError_t launch_prefill_pack(const PackArgs& a, long n_packs, hipStream_t s);
 hipError_t launch_prefill_flash(const FlashArgs& a, hipStream_t s);

@@ -69,3 +69,26 @@ def test_canary_windows_beyond_one_chunk(device, window, kg, d, hq, h, nq):
           flush=True)
     _close(got, ref)
     assert (ref[:, 0] > ref[:, 1]).all() and (ref[:, 1] > ref[:, 2]).all()
+
+
+@pytest.mark.parametrize("window,kg,d,hq,h,nq,bits", [
+    (80, 24, 100, 32, 2, 8, (2, 4, 8)),   # 128 query rows: two passes; groups straddling chunks; padded channels
+    (130, 1, 128, 8, 2, 3, (2, 8)),       # groups of one key; two tiers; 12 rows (a partial row block)
+    (70, 7, 256, 6, 2, 5, (4,)),          # one tier; head size 256
+    (33, 3, 6, 17, 1, 1, (2, 4, 8)),      # 17 rows, 6 channels
+])
+def test_canary_rows_groups_and_tiers_at_their_edges(device, window, kg, d, hq, h, nq, bits):
+    """Query rows past one block of 16 and one pass of 64, K groups that straddle key chunks
+    or hold one key, head sizes that are padded, one to three tiers, and key rows that
+    are not 16-byte aligned; float32 and bf16 queries."""
+    rng = np.random.default_rng(window + d)
+    kref = (rng.standard_normal((2, window, h, d)) * 2).astype(np.float32)
+    wide = torch.zeros(2, window, h, d + 3, device=device)
+    wide[..., 1 : d + 1] = torch.from_numpy(kref).to(device)
+    for dt in (torch.float32, torch.bfloat16):
+        q = torch.from_numpy(rng.standard_normal((2, nq, hq, d)).astype(np.float32)).to(dt)
+        ref = OC.canary_kl(q.float().numpy(), kref, bits, kg, d ** -0.5)
+        for k in (torch.from_numpy(kref).to(device), wide[..., 1 : d + 1]):
+            got = canary_kl(q.to(device), k, bits, kg, d ** -0.5)
+            assert got.shape == (2, len(bits))
+            _close(got, ref)
