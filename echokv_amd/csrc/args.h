@@ -70,8 +70,15 @@ struct StepArgs {
   // its K group over 4 lanes per item (staged dtype, k_group 8 to 64); 0: one
   // workgroup per fin row.
   int fin_parts;
+  // 1: a large step as two launches, fin rows (split, fin_parts > 0) then token rows of 16
+  // channels a lane (head size a multiple of 16, V groups of 16 x 2^j channels, value rows
+  // aligned for 16-byte loads).
+  int wide;
 };
 
+// Token rows from which a step is two launches: both take 15 us at 1500 rows (INT4, H 8, D 128;
+// 1000: 11.0 fused, 13.9 apart; 2100: 19.2 fused, 16.2 apart; 8400: 68, 31).
+constexpr int kWideRows = 1536;
 // Dynamic LDS of a staged fused step, and the largest the launch takes without
 // raising the kernel's limit.
 inline size_t step_staged_lds(int k_group, int dtype) {

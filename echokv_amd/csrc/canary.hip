@@ -50,16 +50,6 @@ __host__ __device__ inline int canary_groups(int C, int kg) {
   return kg == 1 ? 0 : (C + kg - 1) / kg + (C % kg && kg % C ? 1 : 0);
 }
 
-// quant_code's value with the division replaced where that cannot change it: (x - m) * r,
-// r = 1 / s to an ulp or two, is within 255 * 2^-21 of the quotient, so both round to the
-// same code unless the product lies that close to a tie (then, and for NaN, divide).
-__device__ __forceinline__ float code_of(float x, float m, float s, float r, float levels) {
-  const float t = (x - m) * r;
-  float q = __builtin_rintf(t);
-  if (!(fabsf(t - q) < 0.4995f)) q = __builtin_rintf((x - m) / s);
-  return fminf(fmaxf(q, 0.0f), levels);
-}
-
 __device__ __forceinline__ float rows4_sum(float x) {  // over lanes l, l ^ 16, l ^ 32, l ^ 48
   x += __shfl_xor(x, 16, 64);
   return x + __shfl_xor(x, 32, 64);
@@ -182,7 +172,6 @@ __global__ __launch_bounds__(256) void canary_kernel(CanaryArgs a) {
         // The variant's keys as A operands: lane (c, n) holds key 16 kt + n, channels 16 g + 4c + u
         // at step (g, u); queries alike, so a step's four products cover 16 channels in any order.
         f4_t kf[KT][DG];
-        const float levels = (float)((1 << bits) - 1);
 #pragma unroll
         for (int kt = 0; kt < KT; ++kt) {
           const uint32_t* sp = st + ((wave - 1) * L.NG + (wave >= 1 ? (c0 + 16 * kt + n) / a.kg - g0 : 0)) * DP + 4 * c;
@@ -196,7 +185,7 @@ __global__ __launch_bounds__(256) void canary_kernel(CanaryArgs a) {
                 _Float16 s16, m16;
                 float s, m;
                 group_stats(y[u], y[u], bits, s16, m16, s, m);
-                y[u] = code_of(y[u], m, s, __builtin_amdgcn_rcpf(s), levels) * s + m;
+                y[u] = (float)quant_code(y[u], m, s, bits) * s + m;
               }
             } else if (tier) {
               const uint4 sm = *(const uint4*)(sp + 16 * g);
@@ -205,7 +194,10 @@ __global__ __launch_bounds__(256) void canary_kernel(CanaryArgs a) {
               for (int u = 0; u < 4; ++u) {
                 const float s = (float)__builtin_bit_cast(_Float16, (uint16_t)pk[u]);
                 const float m = (float)__builtin_bit_cast(_Float16, (uint16_t)(pk[u] >> 16));
-                y[u] = code_of(y[u], m, s, __builtin_amdgcn_rcpf(s), levels) * s + m;
+                bool tie = false;
+                uint32_t q = quant_code_r(y[u], m, __builtin_amdgcn_rcpf(s), bits, tie);
+                if (tie) q = quant_code(y[u], m, s, bits);
+                y[u] = (float)q * s + m;
               }
             }
             kf[kt][g] = y;

@@ -170,6 +170,19 @@ __device__ __forceinline__ uint32_t quant_code(float x, float m, float s, int bi
   return (uint32_t)q;
 }
 
+// quant_code by r = 1 / s to an ulp (v_rcp_f32) instead of a division, where that gives
+// the same code: (x - m) * r is within 1.8e-7 of the divided value relatively, so within
+// (levels + 1) * 2.4e-7 of it as far as the clamp, and both round to one code unless the
+// product lies that close to a tie. `tie` is set there (at twice the distance), and for
+// infinities and NaN (the comparison fails): take quant_code then.
+__device__ __forceinline__ uint32_t quant_code_r(float x, float m, float r, int bits, bool& tie) {
+#pragma clang fp contract(off)
+  const float levels = (float)((1 << bits) - 1);
+  const float t = (x - m) * r, q = __builtin_rintf(t);
+  tie = tie || !(fabsf(t - q) < 0.5f - (levels + 1.0f) * 4.8e-7f);
+  return (uint32_t)fminf(fmaxf(q, 0.0f), levels);
+}
+
 // Pack four codes (channels 4c..4c+3) little-endian inside bytes.
 __device__ __forceinline__ uint32_t pack4(const uint32_t q[4], int bits) {
   return q[0] | (q[1] << bits) | (q[2] << (2 * bits)) | (q[3] << (3 * bits));

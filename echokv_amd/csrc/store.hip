@@ -575,14 +575,16 @@ __device__ __forceinline__ void fin_staged(const StepArgs& s, long f, typename R
 // dependent divisions per thread, not k_group. The residual words of a deferred
 // row are rewritten by the thread that read that position (if it read the
 // residual there), after its read.
-template <int DT, int TPT>
-__device__ __forceinline__ void fin_split(const StepArgs& s, const FinHead& fh, int part, const Deferred& def,
+// RCP: codes by quant_code_r (large steps, where the divisions are the time; a lone fin
+// row's time is its round trips, and the shorter code is better).
+template <int DT, int TPT, bool RCP>
+__device__ __forceinline__ void fin_split(const StepArgs& s, const FinHead& fh, int part, const Deferred* def,
                                           const int64_t* grow) {
   using V = typename Raw4<DT>::V;
   constexpr long esz = DT == ECHOKV_F32 ? 4 : 2;
   const WriteTokArgs& a = s.w;
   const Lay& L = a.L;
-  const int KG = L.KG;  // = 4 * TPT
+  const int KG = 4 * TPT;  // = L.KG
   const long blk = fh.blk;
   const int grp = fh.grp;
   const long rs_raw = fh.rs;
@@ -661,19 +663,26 @@ __device__ __forceinline__ void fin_split(const StepArgs& s, const FinHead& fh, 
       const long base = j == 0 ? cb[0] : (j == 1 ? cb[1] : (j == 2 ? cb[2] : cb[3]));
       if (base >= 0) {
         uint32_t q[4];
+        bool tie = !RCP;
+        if constexpr (RCP) {
 #pragma unroll
-        for (int e = 0; e < 4; ++e) q[e] = quant_code(x[u][e], mi[e], sc[e], bits);
+          for (int e = 0; e < 4; ++e) q[e] = quant_code_r(x[u][e], mi[e], __builtin_amdgcn_rcpf(sc[e]), bits, tie);
+        }
+        if (tie) {
+#pragma unroll
+          for (int e = 0; e < 4; ++e) q[e] = quant_code(x[u][e], mi[e], sc[e], bits);
+        }
         store_codes4(a.pages + base + (pos % tpc) * rowb + within, pack4(q, bits), bits);
       }
     }
   }
   // Residual K of the deferred rows whose position this thread holds.
-  if (act) {
-    for (int d = 0; d < def.n; ++d) {
-      if (def.row[d] / TPT != r) continue;
+  if (act && def) {
+    for (int d = 0; d < def->n; ++d) {
+      if (def->row[d] / TPT != r) continue;
       float k[4];
-      ld_n<4>(a.key, a.kv_dtype, def.t[d] * a.k_s0 + h * a.k_s1 + 4 * c, k);
-      st_n<4>(a.res.ptr, a.res.dtype, rs_raw * a.res.s0 + (long)def.row[d] * a.res.s1 + h * a.res.s2 + 4 * c, k);
+      ld_n<4>(a.key, a.kv_dtype, def->t[d] * a.k_s0 + h * a.k_s1 + 4 * c, k);
+      st_n<4>(a.res.ptr, a.res.dtype, rs_raw * a.res.s0 + (long)def->row[d] * a.res.s1 + h * a.res.s2 + 4 * c, k);
     }
   }
 }
@@ -682,10 +691,10 @@ template <int DT>
 __device__ __forceinline__ void fin_split_t(const StepArgs& s, const FinHead& fh, int part, const Deferred& def,
                                             const int64_t* grow) {
   switch (s.w.L.KG) {
-    case 8: fin_split<DT, 2>(s, fh, part, def, grow); break;
-    case 16: fin_split<DT, 4>(s, fh, part, def, grow); break;
-    case 32: fin_split<DT, 8>(s, fh, part, def, grow); break;
-    default: fin_split<DT, 16>(s, fh, part, def, grow); break;  // 64 (the host picks this path for 8 to 64)
+    case 8: fin_split<DT, 2, false>(s, fh, part, &def, grow); break;
+    case 16: fin_split<DT, 4, false>(s, fh, part, &def, grow); break;
+    case 32: fin_split<DT, 8, false>(s, fh, part, &def, grow); break;
+    default: fin_split<DT, 16, false>(s, fh, part, &def, grow); break;  // 64 (the host picks this path for 8 to 64)
   }
 }
 
@@ -745,6 +754,147 @@ __global__ __launch_bounds__(kThreads) void write_step_kernel(StepArgs s) {
     return;
   }
   step_token_row(s, (long)blockIdx.x - fin_wgs);
+}
+
+// ---------------------------------------------------------------------------
+// Large steps (thousands of rows: prompts). The chip is full many times over, so what
+// counts is the work per row and how many rows are in flight, not one row's round trips:
+// the fin rows and the token rows are two launches, each with the registers it needs (the
+// fused kernel's fin rows of up to 64 keys leave its token rows 3 waves a SIMD), in
+// the pair's order, so no residual store is handed over and no token row looks through
+// the fin rows. 8155 rows of 3 requests (INT4, H 8, D 128, bf16, 254 fin
+// rows): 66 us fused, 14 + 14 us here (1.6 TB/s of the bytes it cannot do without).
+// ---------------------------------------------------------------------------
+template <int DT, int TPT>
+__global__ __launch_bounds__(kThreads) void fin_rows_kernel(StepArgs s) {
+  __shared__ int64_t grow[4 * TPT];
+  const long f = blockIdx.x / s.fin_parts;
+  const int part = (int)(blockIdx.x % s.fin_parts);
+  const int64_t* row = s.fin + f * (3 + 4 * TPT);
+  const FinHead fh{row[0], row[2], (int)row[1]};
+  if ((int)threadIdx.x < 4 * TPT) grow[threadIdx.x] = row[3 + threadIdx.x];
+  __syncthreads();
+  if (f >= *s.fin_count) return;
+  fin_split<DT, TPT, true>(s, fh, part, nullptr, grow);
+}
+
+// Sixteen consecutive elements by 16-byte loads (aligned).
+template <int DT>
+__device__ __forceinline__ void ld16v(const void* p, long i, float x[16]) {
+  constexpr int per = DT == ECHOKV_F32 ? 4 : 8;
+  uint4 u[16 / per];
+#pragma unroll
+  for (int k = 0; k < 16 / per; ++k)
+    u[k] = *(const uint4*)((const char*)p + (DT == ECHOKV_F32 ? 4 : 2) * i + 16 * k);
+#pragma unroll
+  for (int e = 0; e < 16; ++e) {
+    const uint4& v = u[e / per];
+    const uint32_t w[4] = {v.x, v.y, v.z, v.w};
+    const int k = e % per;
+    if constexpr (DT == ECHOKV_F32) {
+      x[e] = __uint_as_float(w[k]);
+    } else {
+      const uint16_t b = (uint16_t)(w[k >> 1] >> (16 * (k & 1)));
+      if constexpr (DT == ECHOKV_F16) x[e] = (float)__builtin_bit_cast(_Float16, b);
+      else x[e] = bf16_to_f32(b);
+    }
+  }
+}
+
+// One wave per token row, 16 channels a lane (StepArgs::wide: head size a multiple of 16, V
+// groups of 16 x 2^j channels, aligned value rows): a V group is 1 to 16 lanes, a row's
+// codes go out in 4 to 16 bytes a lane. K is read only for the rows that store it (open
+// groups, sealed groups, the K_ref window: a few per request; the fin rows read the others).
+template <int DT>
+__global__ __launch_bounds__(kThreads) void token_rows_kernel(StepArgs s) {
+  const WriteTokArgs& a = s.w;
+  const Lay& L = a.L;
+  const int lane = threadIdx.x & 63;
+  const long t = (long)blockIdx.x * 4 + (threadIdx.x >> 6);
+  if (t >= s.n_rows) return;
+  const int items = L.H * L.D / 16;  // 16-channel pieces of a row
+  auto value_at = [&](int i) {
+    const int h = 16 * i / L.D, d = 16 * i - h * L.D;
+    return t * a.v_s0 + h * a.v_s1 + d;
+  };
+  // The plan and the first pass's values do not depend on one another: one round trip.
+  const long slot = a.tok[t], rslot = a.tok[a.tok_s0 + t];
+  const int64_t sealed = a.tok[2 * a.tok_s0 + t];
+  const long kidx = a.kref ? a.tok[3 * a.tok_s0 + t] : -1;
+  float x[16];
+  ld16v<DT>(a.value, value_at(lane < items ? lane : 0), x);
+  if (slot < 0) return;
+  const long blk = (uint64_t)slot >> 32 ? slot / L.BS : (long)((uint32_t)slot / (uint32_t)L.BS);
+  const int off = (int)(slot - blk * L.BS);
+  if (blk >= L.nb) return;
+  const Hdr hd = load_hdr(a.pages, L, blk);
+  const int bits = tier_of(hd.tag);
+  const long rb = row_base_h(L, blk, hd, off, bits);
+  if (rb < 0) return;  // its chunk id is out of range: nothing is stored
+  const int G = L.D / L.VG;
+  for (int base = 0; base < items; base += 64) {
+    const int i = base + lane < items ? base + lane : 0;
+    const bool act = base + lane < items;
+    if (base > 0) ld16v<DT>(a.value, value_at(i), x);
+    float mn = x[0], mx = x[0];
+#pragma unroll
+    for (int e = 1; e < 16; ++e) {
+      mn = fminf(mn, x[e]);
+      mx = fmaxf(mx, x[e]);
+    }
+    seg_minmax(mn, mx, L.VG / 16);
+    _Float16 s16, m16;
+    float sc, m;
+    group_stats(mn, mx, bits, s16, m16, sc, m);
+    if (!act) continue;
+    const int h = 16 * i / L.D, d = 16 * i - h * L.D;
+    if (d % L.VG == 0) {
+      const long e = ((long)off * L.H + h) * G + d / L.VG;
+      *f16p(a.pages, blk * L.stride + L.o_vs + 2 * e) = s16;
+      *f16p(a.pages, blk * L.stride + L.o_vm + 2 * e) = m16;
+    }
+    const float r = __builtin_amdgcn_rcpf(sc);
+    uint32_t q[16];
+    bool tie = false;
+#pragma unroll
+    for (int e = 0; e < 16; ++e) q[e] = quant_code_r(x[e], m, r, bits, tie);
+    if (tie) {
+#pragma unroll
+      for (int e = 0; e < 16; ++e) q[e] = quant_code(x[e], m, sc, bits);
+    }
+    uint8_t* dst = a.pages + rb + L.H * L.D * bits / 8 + 2 * i * bits;
+    if (bits == 4) {
+      *(uint2*)dst = uint2{pack4(q, 4) | pack4(q + 4, 4) << 16, pack4(q + 8, 4) | pack4(q + 12, 4) << 16};
+    } else if (bits == 8) {
+      *(uint4*)dst = uint4{pack4(q, 8), pack4(q + 4, 8), pack4(q + 8, 8), pack4(q + 12, 8)};
+    } else {
+      *(uint32_t*)dst = pack4(q, 2) | pack4(q + 4, 2) << 8 | pack4(q + 8, 2) << 16 | pack4(q + 12, 2) << 24;
+    }
+  }
+  if (rslot < 0 && sealed == 0 && kidx < 0) return;
+  // K: residual (open group), codes under the sealed stats, K_ref ring; four channels at a time.
+  const int quads = L.D / 4;
+#pragma unroll 1
+  for (int i = lane; i < L.H * quads; i += 64) {
+    const int h = i / quads, c = i % quads;
+    float k[4];
+    ld_n<4>(a.key, a.kv_dtype, t * a.k_s0 + h * a.k_s1 + 4 * c, k);
+    if (rslot >= 0 && rslot < a.res.rows)
+      st_n<4>(a.res.ptr, a.res.dtype, rslot * a.res.s0 + (long)(off % L.KG) * a.res.s1 + h * a.res.s2 + 4 * c, k);
+    if (sealed != 0) {
+      const long se = ((long)(off / L.KG) * L.H + h) * L.D + 4 * c;
+      uint32_t kq[4];
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+        kq[e] = quant_code(k[e], (float)*f16p(a.pages, blk * L.stride + L.o_km + 2 * (se + e)),
+                           (float)*f16p(a.pages, blk * L.stride + L.o_ks + 2 * (se + e)), bits);
+      store_codes4(a.pages + rb + (long)h * (L.D * bits / 8) + c * (bits / 2), pack4(kq, bits), bits);
+    }
+    if (kidx >= 0) {
+#pragma unroll
+      for (int e = 0; e < 4; ++e) a.kref[kidx * a.kref_s0 + h * a.kref_s1 + 4 * c + e] = k[e];
+    }
+  }
 }
 
 // ---------------------------------------------------------------------------
@@ -1009,7 +1159,33 @@ hipError_t launch_finalize_k(const FinArgs& a, long rows, hipStream_t s) {
   hipLaunchKernelGGL(finalize_k_kernel, dim3((unsigned)rows), dim3(kThreads), 0, s, a);
   return hipGetLastError();
 }
+template <int DT>
+static hipError_t launch_fin_rows(const StepArgs& a, hipStream_t s) {
+  const dim3 grid((unsigned)(a.fin_grid * a.fin_parts));
+  switch (a.w.L.KG) {
+    case 8: hipLaunchKernelGGL((fin_rows_kernel<DT, 2>), grid, dim3(kThreads), 0, s, a); break;
+    case 16: hipLaunchKernelGGL((fin_rows_kernel<DT, 4>), grid, dim3(kThreads), 0, s, a); break;
+    case 32: hipLaunchKernelGGL((fin_rows_kernel<DT, 8>), grid, dim3(kThreads), 0, s, a); break;
+    default: hipLaunchKernelGGL((fin_rows_kernel<DT, 16>), grid, dim3(kThreads), 0, s, a); break;  // 64
+  }
+  return hipGetLastError();
+}
+template <int DT>
+static hipError_t launch_large_step(const StepArgs& a, hipStream_t s) {
+  if (a.fin_grid > 0) {
+    const hipError_t e = launch_fin_rows<DT>(a, s);
+    if (e != hipSuccess) return e;
+  }
+  hipLaunchKernelGGL(token_rows_kernel<DT>, dim3((unsigned)((a.n_rows + 3) / 4)), dim3(kThreads), 0, s, a);
+  return hipGetLastError();
+}
+
 hipError_t launch_write_step(const StepArgs& a, hipStream_t s) {
+  if (a.wide) {
+    if (a.w.kv_dtype == ECHOKV_F16) return launch_large_step<ECHOKV_F16>(a, s);
+    if (a.w.kv_dtype == ECHOKV_BF16) return launch_large_step<ECHOKV_BF16>(a, s);
+    return launch_large_step<ECHOKV_F32>(a, s);
+  }
   const size_t lds = a.staged < 0 || a.fin_parts > 0 ? 0 : step_staged_lds(a.w.L.KG, a.staged);
   const long fin_wgs = a.fin_parts > 0 ? a.fin_grid * a.fin_parts : a.fin_grid;
   hipLaunchKernelGGL(write_step_kernel, dim3((unsigned)(fin_wgs + a.n_rows)), dim3(kThreads), lds, s, a);

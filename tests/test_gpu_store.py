@@ -315,3 +315,70 @@ def test_aligned_pages_hold_the_same_bytes_and_decode_the_same(device, name):
         b = dec.decode_attention(plain, q, table, lens, s.d ** -0.5, blocks_per_split=bps)
         torch.cuda.synchronize()
         assert torch.equal(a, b), f"{name} bps={bps}"
+
+
+@pytest.mark.parametrize("h,d,bs,kg,vg,dt", [
+    (8, 128, 16, 16, 32, torch.bfloat16),
+    (3, 64, 32, 32, 64, torch.float16),     # 12 lanes of a wave
+    (5, 256, 64, 32, 16, torch.float32),    # two passes of a wave, V groups of one lane
+    (2, 128, 128, 64, 128, torch.bfloat16),  # V groups of 8 lanes
+    (4, 48, 48, 16, 16, torch.float16),     # block size not a power of two
+    (4, 96, 16, 8, 24, torch.bfloat16)])    # V groups that are not lanes: the fused launch
+@pytest.mark.parametrize("bits", [2, 4, 8])
+def test_large_steps_equal_the_pair(device, h, d, bs, kg, vg, dt, bits):
+    """Steps of more than kWideRows (1536) token rows -- fin rows and token rows as two
+    launches of their own kernels -- leave exactly the bytes, residual and K_ref ring of
+    finalize_k then write_tokens: prompts, groups completed from the residual and the step's
+    keys, evicted (sealed) groups continued, released slots taken again in the same
+    step, rows without a slot, values as slices of a wider tensor."""
+    from echokv_amd.kernels.write import finalize_k, write_step, write_tokens
+    from echokv_amd.tiered_cache import TieredKVCache, TieredLayout
+    from echokv_amd.write_plan import SharedState, stage_plan
+
+    rng = np.random.default_rng(d + kg)
+    n_seq, half, per = 40, 20, 90
+    nb_seq = -(-(4 * per) // bs)
+    nb = n_seq * nb_seq + 8
+    table = rng.permutation(nb)[: n_seq * nb_seq].reshape(n_seq, nb_seq)
+    layout = TieredLayout(h, d, bs, 8, kg, vg)
+    page = bs * TieredLayout.per_token_bytes(h, d, 8, kg, vg)
+    stores, krefs = [], []
+    for _ in range(2):
+        shared = SharedState(nb, bs, kg, 24, kref_window=64, device=device)
+        stores.append(TieredKVCache(layout, torch.zeros(nb, page, dtype=torch.uint8, device=device),
+                                    residual=torch.zeros(25, kg, h, d, dtype=dt, device=device), shared=shared))
+        krefs.append(torch.zeros(64, h, d, device=device))
+    lens = np.zeros(n_seq, np.int64)
+    gen = torch.Generator(device=device)
+    gen.manual_seed(d)
+    for step, seqs in enumerate((range(half), range(half, n_seq), range(half), range(half - 4, n_seq - 4))):
+        parts = []
+        for s in seqs:
+            n = int(rng.integers(per - 12, per))
+            p = np.arange(lens[s], lens[s] + n)
+            parts.append(table[s][p // bs] * bs + p % bs)
+            lens[s] += n
+        slots = np.concatenate(parts)
+        slots[:: 97] = -1 if step == 3 else slots[:: 97]  # rows without a slot
+        assert slots.size >= 1536
+        kv = torch.randn(slots.size, 3, h, d, device=device, generator=gen).to(dt)
+        if step == 2:
+            kv = (8 * kv).round()  # whole numbers: codes that lie on rounding ties
+        for store, kref, fused in zip(stores, krefs, (True, False)):
+            plan = store.planner.plan(torch.from_numpy(slots))
+            opened = store.prepare(plan, bits)
+            store.shared.commit(plan)
+            meta, extra = stage_plan(plan, device, opened)
+            store.shared.apply_res_map(*extra[:4])
+            if opened is not None:
+                store.write_headers(extra[4], extra[5])
+            if fused:
+                write_step(store, kv[:, 0], kv[:, 1], meta, kref)
+            else:
+                finalize_k(store, kv[:, 0], meta)
+                write_tokens(store, kv[:, 0], kv[:, 1], meta, kref)
+        torch.cuda.synchronize()
+        assert torch.equal(stores[0].pages, stores[1].pages), f"pages differ after step {step}"
+        assert torch.equal(stores[0].res_k, stores[1].res_k), f"residual differs after step {step}"
+        assert torch.equal(krefs[0], krefs[1]), f"K_ref differs after step {step}"
+    assert stores[0].sealed_groups > 0
