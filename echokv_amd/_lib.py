@@ -18,7 +18,7 @@ import torch
 LIB_PATH = Path(__file__).resolve().parent / "libechokv.so"
 
 F32, F16, BF16 = 0, 1, 2
-DECODE_BATCH_INVARIANT = 1
+DECODE_BATCH_INVARIANT, DECODE_SHORT_SPLITS = 1, 4
 DTYPES = {torch.float32: F32, torch.float16: F16, torch.bfloat16: BF16}
 
 EXPORTS = (

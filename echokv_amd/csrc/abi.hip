@@ -229,7 +229,7 @@ int decode_run(const echokv_layout* L, const uint8_t* pages, const int64_t* bloc
   if (!dtype_ok(q_dtype) || !dtype_ok(out_dtype)) return ECHOKV_EDTYPE;
   if (num_seqs < 0 || num_splits <= 0 || blocks_per_split <= 0 || !res_ok(res)) return ECHOKV_EINVAL;
   if (tier != 2 && tier != 4 && tier != 8) return ECHOKV_EINVAL;
-  if (flags & ~ECHOKV_DECODE_BATCH_INVARIANT) return ECHOKV_EINVAL;
+  if (flags & ~(ECHOKV_DECODE_BATCH_INVARIANT | ECHOKV_DECODE_SHORT_SPLITS)) return ECHOKV_EINVAL;
   if (tier_mask && !(flags & ECHOKV_DECODE_BATCH_INVARIANT)) return ECHOKV_EINVAL;  // tier passes: split schedule
   if (num_seqs == 0) return ECHOKV_OK;
   if (!pages || !block_res || !res_group || !query || !block_table || !seq_lens || !out) return ECHOKV_EINVAL;
@@ -253,7 +253,7 @@ int decode_run(const echokv_layout* L, const uint8_t* pages, const int64_t* bloc
   a.lens = seq_lens;
   a.scale_log2 = softmax_scale * 1.4426950408889634f;
   a.num_splits = num_splits;
-  a.bps = blocks_per_split;
+  a.sp = ek::make_splits(num_splits, blocks_per_split, L->block_size, flags & ECHOKV_DECODE_SHORT_SPLITS);
   a.num_seqs = num_seqs;
   a.tier = tier;
   a.tier0 = tier;
@@ -313,7 +313,7 @@ int decode_run(const echokv_layout* L, const uint8_t* pages, const int64_t* bloc
       e = ek::launch_merge_balanced(a, (hipStream_t)stream);
     } else {
       ek::MergeArgs m{acc, ml, seq_lens, q_rows, out, o_s0, o_s1, out_dtype, num_q_heads, L->head_size,
-                      L->block_size, num_splits, blocks_per_split, num_seqs * num_q_heads, gqa, a.g0, a.gs};
+                      L->block_size, num_splits, a.sp, num_seqs * num_q_heads, gqa, a.g0, a.gs};
       e = mfma ? ek::launch_merge(m, num_seqs, (hipStream_t)stream) : ek::launch_merge_any(m, (hipStream_t)stream);
     }
     if (e != hipSuccess) return ECHOKV_ELAUNCH;
@@ -352,7 +352,7 @@ int echokv_decode_static(const echokv_layout* L, const uint8_t* pages, const int
 int64_t echokv_decode_workspace_rows(const echokv_layout* L, int32_t num_q_heads, int32_t q_dtype,
                                      int64_t num_seqs, int32_t num_splits, int32_t flags) {
   if (!lay_ok(L) || num_q_heads <= 0 || num_q_heads % L->num_kv_heads || num_seqs < 0 || num_splits <= 0 ||
-      !dtype_ok(q_dtype) || (flags & ~ECHOKV_DECODE_BATCH_INVARIANT))
+      !dtype_ok(q_dtype) || (flags & ~(ECHOKV_DECODE_BATCH_INVARIANT | ECHOKV_DECODE_SHORT_SPLITS)))
     return -1;
   const int64_t split_rows = num_seqs * num_splits;
   if (!decode_mfma(L) || (flags & ECHOKV_DECODE_BATCH_INVARIANT) || num_seqs == 0) return split_rows;

@@ -164,6 +164,30 @@ struct DenseArgs {
   int out_dtype;
 };
 
+// The split schedule's split sizes, in blocks: bps, or what num_splits splits of the
+// sequence need. With ECHOKV_DECODE_SHORT_SPLITS a sequence of up to cut4 = bps blocks is cut
+// in four and one of up to cut3 = 1.5 bps in three, down to min blocks (128 tokens): a split
+// is a serial chain of tiles, and such sequences would be one or two of them however
+// idle the chip is (one 1337-token request, 64-token blocks, INT4: 72 us in two splits of
+// 1024 tokens, 45 in three). The rule looks at the sequence alone, so it also holds where the
+// batch fills the chip, and there every further split costs about 12 us of one
+// workgroup: cutting longer sequences finer too takes 128 x 2048 tokens from 129 us (1024 a
+// split) to 132 (512) or 147 (256), so they keep bps. cut4 = cut3 = min = 0: bps alone.
+struct Splits {
+  int num, bps, cut4, cut3, min;
+};
+__host__ __device__ inline Splits make_splits(int num, int bps, int block_size, bool short_splits) {
+  if (!short_splits) return Splits{num, bps, 0, 0, 0};
+  return Splits{num, bps, bps, bps > (1 << 30) ? bps : bps + bps / 2, (127 + block_size) / block_size};
+}
+__host__ __device__ inline int split_blocks(const Splits& s, int nb) {
+  int b = nb <= s.cut4 ? (nb + 3) >> 2 : (nb <= s.cut3 ? (nb + 2) / 3 : s.bps);
+  b = b > s.min ? b : s.min;
+  b = b < s.bps ? b : s.bps;
+  const int per = (nb + s.num - 1) / s.num;
+  return b > per ? b : per;
+}
+
 struct DecodeArgs {
   Lay L;
   const uint8_t* pages;
@@ -183,7 +207,8 @@ struct DecodeArgs {
   const int64_t* bt_rows;
   const int64_t* lens;
   float scale_log2;  // softmax scale * log2(e)
-  int num_splits, bps;
+  int num_splits;
+  Splits sp;  // the split schedule
   long num_seqs;
   int tier;    // the layer's tier: selects the kernel specialised for it (2, 4 or 8)
   // Tier passes (split schedule): null, or the layer's tiers with live blocks as a
@@ -225,7 +250,8 @@ struct MergeArgs {
   const int64_t* q_rows;
   void* out;
   long o_s0, o_s1;
-  int out_dtype, hq, D, BS, num_splits, bps;
+  int out_dtype, hq, D, BS, num_splits;
+  Splits sp;
   long rows;  // num_seqs * hq
   int gqa, g0, gs;  // rows of query heads g0 .. g0 + gs - 1 of each KV head only
 };

@@ -40,7 +40,7 @@
 // than 2^8 (probabilities stay <= 256, far inside fp16).
 //
 // A split covers max(blocks_per_split, ceil(blocks / num_splits)) blocks of
-// the sequence's own length, so results do not depend on the rest of the
+// the sequence's own length, fewer for short sequences (split_blocks), so results do not depend on the rest of the
 // batch; a second kernel merges the splits in order (log-sum-exp, log2 units).
 #include "items.h"
 
@@ -1286,20 +1286,21 @@ __device__ __forceinline__ uint64_t rl64(uint64_t v, int lane) {
   return (uint64_t)rl((uint32_t)v, lane) | ((uint64_t)rl((uint32_t)(v >> 32), lane) << 32);
 }
 
-// Blocks per split of a sequence of n_blocks blocks:
-// max(blocks_per_split, ceil(blocks / num_splits)).
-__device__ __forceinline__ int split_blocks(const DecodeArgs& a, int n_blocks) {
-  const int per = (n_blocks + a.num_splits - 1) / a.num_splits;
-  return a.bps > per ? a.bps : per;
+// Inclusive prefix sum over the wave's lanes by DPP: row_shr 1, 2, 4, 8 inside rows of 16,
+// then each row's last lane to the rows after it (row_bcast 15, 31). On the start-up
+// chain of every workgroup: six dependent lane permutes through LDS before.
+template <int CTRL, int ROWS>
+__device__ __forceinline__ int dpp_add(int x) {
+  return x + __builtin_amdgcn_update_dpp(0, x, CTRL, ROWS, 0xF, false);
 }
-
 __device__ __forceinline__ int wave_incl_scan(int x, int lane) {
-#pragma unroll
-  for (int d = 1; d < 64; d <<= 1) {
-    const int y = __shfl_up(x, d, 64);
-    if (lane >= d) x += y;
-  }
-  return x;
+  (void)lane;
+  x = dpp_add<0x111, 0xF>(x);
+  x = dpp_add<0x112, 0xF>(x);
+  x = dpp_add<0x114, 0xF>(x);
+  x = dpp_add<0x118, 0xF>(x);
+  x = dpp_add<0x142, 0xA>(x);
+  return dpp_add<0x143, 0xC>(x);
 }
 
 // Inclusive prefixes over sequences [s0, s0 + 64), one per lane, of the
@@ -1311,7 +1312,7 @@ __device__ __forceinline__ int scan_chunk(const DecodeArgs& a, long s0, int lane
   int x = 0;
   if (len > 0) {
     const int nb = (len + a.L.BS - 1) >> a.bs_shift;
-    const int bps = split_blocks(a, nb);
+    const int bps = split_blocks(a.sp, nb);
     x = (((nb + bps - 1) / bps - 1) << 7) | 1;
   }
   return wave_incl_scan(x, lane);
@@ -1746,7 +1747,7 @@ __global__ __launch_bounds__(64 * kHeadsPerGroup, (BITS == 8 || QLO) ? 2 : 3) vo
   int split;
   if (!locate(a, item / n_hg, lane, incl0, seq, split)) return;
   const int n_blocks = ((int)a.lens[seq] + a.L.BS - 1) >> a.bs_shift;
-  const int bps = split_blocks(a, n_blocks);
+  const int bps = split_blocks(a.sp, n_blocks);
   const int b_start = split * bps;
   const int b_end = b_start + bps < n_blocks ? b_start + bps : n_blocks;
   // INT2 splits take the range-share wave priorities too (cfg2 INT2 layer-step
@@ -2128,8 +2129,7 @@ __global__ __launch_bounds__(256) void merge_kernel(MergeArgs a) {
   const int seq_len = (int)a.lens[seq];
   if (seq_len <= 0) return;
   const int n_blocks = (seq_len + a.BS - 1) / a.BS;
-  const int per = (n_blocks + a.num_splits - 1) / a.num_splits;
-  const int bps = a.bps > per ? a.bps : per;
+  const int bps = split_blocks(a.sp, n_blocks);
   const int used = (n_blocks + bps - 1) / bps;
   merge_row<D>(a, row, seq, head, used, lane);
 }

@@ -7,7 +7,7 @@
 //
 // One workgroup per (sequence, KV head, split, group of query heads) in fp32 arithmetic,
 // the split schedule of the MFMA kernels (splits of max(blocks_per_split, ceil(blocks /
-// num_splits)) blocks, so a sequence's result does not depend on its batch) and
+// num_splits)) blocks, fewer for short sequences, so a sequence's result does not depend on its batch) and
 // the same workspace rows: acc [S, Hq, splits, D] unnormalized, ml (running max
 // in log2 units, sum). Keys and values go from codes to registers to products: a lane
 // holds 8 channels of its query heads and of O, a row of 16 lanes (8 up to head size
@@ -86,8 +86,7 @@ __global__ __launch_bounds__(kDecThreads, GS * NO == 1 ? 4 : 2) void decode_any_
   const long seq_len = a.lens[seq];
   if (seq_len <= 0) return;
   const long n_blocks = (seq_len + L.BS - 1) / L.BS;
-  const long per = (n_blocks + a.num_splits - 1) / a.num_splits;
-  const long bps = a.bps > per ? a.bps : per;
+  const long bps = split_blocks(a.sp, (int)n_blocks);
   const long b0 = sp * bps;
   if (b0 >= n_blocks) return;
   const int t_begin = (int)(b0 * L.BS);
@@ -463,8 +462,7 @@ __global__ __launch_bounds__(256) void merge_any_kernel(MergeArgs a) {
   const long seq_len = a.lens[seq];
   if (seq_len <= 0) return;
   const long n_blocks = (seq_len + a.BS - 1) / a.BS;
-  const long per = (n_blocks + a.num_splits - 1) / a.num_splits;
-  const long bps = a.bps > per ? a.bps : per;
+  const long bps = split_blocks(a.sp, (int)n_blocks);
   const int used = (int)((n_blocks + bps - 1) / bps);
   const long base = row * a.num_splits;
   const int D = a.D;

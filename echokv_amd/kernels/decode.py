@@ -9,8 +9,8 @@ writes each sequence's output row. Layouts those kernels are not built for
 groups that are not powers of two, more than 4 chunks per page) take an fp32
 kernel with the same split schedule (``echokv_amd/csrc/decode_any.hip``). A sequence is cut into at most
 ``num_splits`` splits of ``max(blocks_per_split, ceil(blocks / num_splits))``
-blocks, a function of its own length, so its result does not depend on the
-rest of the batch.
+blocks -- a sequence of up to 1.5 ``blocks_per_split`` blocks into three or four --
+a function of its own length, so its result does not depend on the rest of the batch.
 """
 
 from __future__ import annotations
@@ -20,6 +20,7 @@ import torch
 from echokv_amd import _lib
 
 BLOCKS_PER_SPLIT = 16
+SHORT_SPLITS = 4  # a short sequence's splits (csrc/args.h, split_blocks); fewer are not cut finer
 MAX_SPLITS = 64  # default cap: more, shorter splits keep every CU busy at small batch
 
 
@@ -78,7 +79,8 @@ def decode_attention(
     of the store's blocks are stored at. Blocks of other tiers are read correctly
     either way. With ``batch_invariant`` (the default, as the reference's decode) each
     sequence is split by its own length, so its result does not depend on the rest
-    of the batch; ``batch_invariant=False`` spreads the batch's blocks evenly over
+    of the batch (calls that name ``num_splits`` themselves: of calls naming at least
+    ``SHORT_SPLITS``); ``batch_invariant=False`` spreads the batch's blocks evenly over
     every workgroup the GPU holds instead (faster on uneven batches; a sequence's
     result then depends on the rest of the batch through float rounding).
     ``tier_mask``: for a layer holding blocks at several tiers, each tier's blocks
@@ -93,8 +95,17 @@ def decode_attention(
     _lib.require_device(query, block_table, seq_lens, store.pages)
     s = seq_lens.shape[0]
     hq, d = query.shape[1], query.shape[2]
+    # Short sequences are cut finer where the splits they need are there in every call: a
+    # caller's num_splits of at least SHORT_SPLITS, or the call's own count and workspace. A
+    # caller's workspace with the call's own count keeps the count it was sized for.
+    flags = _lib.DECODE_BATCH_INVARIANT if batch_invariant else 0
     if num_splits is None:
         num_splits = default_splits(block_table, L.block_size, blocks_per_split, max_len)
+        if batch_invariant and workspace is None:
+            num_splits = max(num_splits, SHORT_SPLITS)
+            flags |= _lib.DECODE_SHORT_SPLITS
+    elif batch_invariant and num_splits >= SHORT_SPLITS:
+        flags |= _lib.DECODE_SHORT_SPLITS
     if query.stride(2) != 1:
         query = query.contiguous()
     if block_table.dtype != torch.int32 or block_table.stride(1) != 1:
@@ -112,7 +123,6 @@ def decode_attention(
             raise ValueError(f"workspace must be a (acc, ml) pair or 'static', got {workspace!r}")
         acc = ml = None
     else:
-        flags = _lib.DECODE_BATCH_INVARIANT if batch_invariant else 0
         rows = workspace_rows(store, hq, query.dtype, s, num_splits, flags)
         if workspace is None:
             acc = torch.empty(rows, hq, d, device=dev, dtype=torch.float32)
@@ -141,7 +151,7 @@ def decode_attention(
             _lib.byref(res), _lib.ptr(query), query.stride(0), query.stride(1), _lib.dtype_code(query), hq,
             _lib.ptr(q_rows), _lib.ptr(block_table), block_table.stride(0), _lib.ptr(bt_rows), _lib.ptr(lens), s,
             float(softmax_scale), int(num_splits), int(blocks_per_split), int(tier), _lib.ptr(tier_mask),
-            _lib.DECODE_BATCH_INVARIANT if batch_invariant else 0)
+            flags)
     tail = (_lib.ptr(out), out.stride(0), out.stride(1), _lib.dtype_code(out), _lib.stream())
     if static:
         _lib.call("echokv_decode_static", *head, *tail)

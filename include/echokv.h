@@ -36,7 +36,7 @@ enum {
 };
 
 /* echokv_decode flags. */
-enum { ECHOKV_DECODE_BATCH_INVARIANT = 1 };
+enum { ECHOKV_DECODE_BATCH_INVARIANT = 1, ECHOKV_DECODE_SHORT_SPLITS = 4 };
 
 /* One layer's page layout (echokv_vllm/tiered_cache.py:76-147, TieredLayout):
  * header [0, block_size); V scale/min fp16 [block_size, H, D/v_group];
@@ -137,7 +137,10 @@ int echokv_store_blocks(const echokv_layout* L, uint8_t* pages, const int64_t* b
  * written directly, the others merged from partials. With flags &
  * ECHOKV_DECODE_BATCH_INVARIANT: split-KV with splits of
  * max(blocks_per_split, ceil(blocks / num_splits)) blocks of the sequence's own
- * length, so a sequence's result does not depend on the rest of the batch. tier
+ * length, so a sequence's result does not depend on the rest of the batch; with
+ * ECHOKV_DECODE_SHORT_SPLITS too, a sequence of up to blocks_per_split blocks is cut in
+ * four and one of up to 1.5 times as many in three (splits of at least 128 tokens, at most
+ * num_splits: give 4 or more), still by its own length. tier
  * (2, 4 or 8) selects the kernel specialised for the layer's tier; blocks stored at
  * another tier, and each block's open K group, are still read correctly on a slower
  * path. tier_mask (device int32, or NULL) names the tiers the layer holds blocks at,

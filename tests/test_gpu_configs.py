@@ -305,6 +305,40 @@ def test_cfg4_gqa8_long_context_split_paths(device):
     assert -(-nblk // 4) > 64 and -(-nblk // -(-nblk // 200)) > 64
 
 
+@pytest.mark.parametrize("d,vg", [(128, 32), (64, 32), (96, 24)])
+def test_short_sequences_are_cut_by_their_own_length(device, d, vg):
+    """The finer splits of short sequences (up to 16 blocks of 64 tokens in four, up to 24 in
+    three, 128 tokens at least): every edge of the rule against the oracle, the same bits
+    alone and in the batch without num_splits and for any num_splits of 4 and more where the
+    rule decides, and a caller's workspace with no num_splits still taken."""
+    bs, h, gqa = 64, 2, 4
+    lens = np.array([1, 64, 65, 128, 129, 500, 512, 513, 15 * 64, 16 * 64, 16 * 64 + 1, 24 * 64, 24 * 64 + 1, 26 * 64])
+    store, table = build_layer(device, lens, 4, h=h, d=d, bs=bs, kg=32, vg=vg, mem_bits=4, seed=17)
+    ref_ps = oracle_view(store)
+    gen = torch.Generator(device=device)
+    gen.manual_seed(170)
+    q = torch.randn(len(lens), gqa * h, d, device=device, generator=gen).half()
+    table_d, lens_d = torch.from_numpy(table).to(device, torch.int32), torch.from_numpy(lens).to(device)
+    ref = OA.decode_attention(ref_ps, q.float().cpu().numpy(), table, lens, d ** -0.5, vectorized=True)
+    full = dec.decode_attention(store, q, table_d, lens_d, d ** -0.5)
+    check(f"short splits D{d}", full, ref)
+    short = torch.from_numpy(lens <= 24 * bs).to(device)
+    for ns in (4, 7, 32):
+        got = dec.decode_attention(store, q, table_d, lens_d, d ** -0.5, num_splits=ns)
+        check(f"short splits D{d} num_splits {ns}", got, ref)
+        assert torch.equal(got[short], full[short])
+    for ns in (1, 3):
+        check(f"short splits D{d} num_splits {ns}", dec.decode_attention(store, q, table_d, lens_d, d ** -0.5,
+                                                                         num_splits=ns), ref)
+    for i, n in enumerate(lens.tolist()):
+        alone = dec.decode_attention(store, q[i : i + 1], table_d[i : i + 1, : -(-n // bs)].contiguous(),
+                                     lens_d[i : i + 1], d ** -0.5)
+        assert torch.equal(alone[0], full[i]), n
+    two = (torch.empty(len(lens) * 2, gqa * h, d, device=device), torch.empty(len(lens) * 2, gqa * h, 2, device=device))
+    check(f"short splits D{d} workspace of the old count",
+          dec.decode_attention(store, q, table_d, lens_d, d ** -0.5, workspace=two), ref)
+
+
 @pytest.mark.parametrize("bits", [8, 4, 2])
 def test_balanced_cost_ranges_at_every_boundary_position(device, bits):
     """The balanced schedule's ranges of equal cost (a live sequence costs its blocks
