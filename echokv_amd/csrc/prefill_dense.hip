@@ -41,6 +41,8 @@ namespace {
 typedef float f16v_t __attribute__((ext_vector_type(16)));
 typedef int v8i_t __attribute__((ext_vector_type(8)));
 typedef int v4i_t __attribute__((ext_vector_type(4)));
+typedef uint32_t u4_t __attribute__((ext_vector_type(4)));
+typedef uint32_t u4_any_t __attribute__((ext_vector_type(4), aligned(2)));  // query / output rows: any alignment
 
 // K lo is stored as e4m3 of (x - hi) * 2^kLoShift; |x - hi| <= 2^-11 |x|, so the
 // stored value stays within |x| (e4m3 holds up to 448; larger ones saturate).
@@ -248,12 +250,12 @@ __global__ __launch_bounds__(64 * kDenseWaves) void flash_kernel(FlashArgs a) {
   // Items (query tile, head) are dealt to the 8 XCDs round-robin by dispatch
   // order; map dispatch b so that XCD b % 8 takes a contiguous run of items:
   // the query tiles of one request and head run on one XCD and share its L2.
-  const long N = (long)a.n_qtiles * a.H;
-  const long b = blockIdx.x;
-  const long q8 = N / 8;
-  const long item = b < 8 * q8 ? (b % 8) * q8 + b / 8 : b;
-  const int h = (int)(item / a.n_qtiles);
-  const int qt = (int)(item % a.n_qtiles);
+  const uint32_t N = (uint32_t)a.n_qtiles * a.H;  // at most INT32_MAX, checked on the host
+  const uint32_t b = blockIdx.x;
+  const uint32_t q8 = N / 8;
+  const uint32_t item = b < 8 * q8 ? (b % 8) * q8 + b / 8 : b;
+  const int h = (int)(item / (uint32_t)a.n_qtiles);
+  const int qt = (int)(item % (uint32_t)a.n_qtiles);
 
   const int32_t* td = a.qtiles + qt * 5;
   const long q_row0 = td[0];
@@ -309,47 +311,70 @@ __global__ __launch_bounds__(64 * kDenseWaves) void flash_kernel(FlashArgs a) {
     if (i < n_kt) issue(i);
 
   // Query fragments (B operand of S^T): row r, channels 16 s + 8 hh .. +8 as fp16;
-  // for K lo, channels 64 c + 32 hh .. +32 as e4m3.
+  // for K lo, channels 64 c + 32 hh .. +32 as e4m3: what the two half-waves hold of steps
+  // 4c .. 4c + 3, exchanged. Every load of the row is requested before the first is
+  // converted (QLO: float32 rows, else 16-bit ones): a round trip to memory for every 8
+  // channels was most of the 20 us a workgroup spent outside its tiles (a 1500-token
+  // prompt 71.9 -> 58.1 us, 16 chunks of 512 tokens over up to 4096 keys 471 -> 415 us).
   h8_t qf[NS], ql[QLO ? NS : 1];
   v8i_t qe[NLO];
   {
-    const int tok = rv ? r / gqa : 0;
-    const int qh = h * gqa + (rv ? r % gqa : 0);
-    const long qb = (q_row0 + tok) * a.q_s0 + (long)qh * a.q_s1 + 8 * hh;
+    constexpr int QW = QLO ? 2 : 1;  // 16-byte words of 8 channels
+    u4_t raw[NS][QW];
 #pragma unroll
-    for (int c = 0; c < NLO; ++c) {
+    for (int s = 0; s < NS; ++s)
 #pragma unroll
-      for (int u = 0; u < 4; ++u) {
-        float x[8];
-        if (rv) {
-          ld_n<8>(a.q, a.q_dtype, qb - 8 * hh + 64 * c + 32 * hh + 8 * u, x);
-        } else {
+      for (int w = 0; w < QW; ++w) raw[s][w] = u4_t{};
+    if (active) {
+      const int rc = rv ? r : n_rows - 1;
+      const long qb = (q_row0 + rc / gqa) * a.q_s0 + (long)(h * gqa + rc % gqa) * a.q_s1 + 8 * hh;
+      const uint8_t* qp = (const uint8_t*)a.q + qb * (QLO ? 4 : 2);
 #pragma unroll
-          for (int e = 0; e < 8; ++e) x[e] = 0.f;
-        }
+      for (int s = 0; s < NS; ++s)
 #pragma unroll
-        for (int e = 0; e < 8; ++e) x[e] = fminf(fmaxf(x[e], -kLoMax), kLoMax);
-#pragma unroll
-        for (int w = 0; w < 2; ++w) {
-          const int lo2 = __builtin_amdgcn_cvt_pk_fp8_f32(x[4 * w], x[4 * w + 1], 0, false) & 0xffff;
-          const int hi2 = __builtin_amdgcn_cvt_pk_fp8_f32(x[4 * w + 2], x[4 * w + 3], 0, false) & 0xffff;
-          qe[c][2 * u + w] = lo2 | (hi2 << 16);
-        }
-      }
+        for (int w = 0; w < QW; ++w) raw[s][w] = *(const u4_any_t*)(qp + 32 * QW * s + 16 * w);
     }
+    const bool bf = a.q_dtype == ECHOKV_BF16;
+    int e8[NS][2];
 #pragma unroll
     for (int s = 0; s < NS; ++s) {
       float x[8];
-      if (rv) {
-        ld_n<8>(a.q, a.q_dtype, qb + 16 * s, x);
-      } else {
+      if constexpr (QLO) {
 #pragma unroll
-        for (int e = 0; e < 8; ++e) x[e] = 0.f;
+        for (int e = 0; e < 8; ++e) x[e] = __uint_as_float(raw[s][e >> 2][e & 3]);
+      } else if (bf) {
+#pragma unroll
+        for (int e = 0; e < 8; ++e) x[e] = bf16_to_f32((uint16_t)(raw[s][0][e >> 1] >> (16 * (e & 1))));
+      } else {
+        const h8_t v = __builtin_bit_cast(h8_t, raw[s][0]);
+#pragma unroll
+        for (int e = 0; e < 8; ++e) x[e] = (float)v[e];
       }
 #pragma unroll
       for (int e = 0; e < 8; ++e) {
+        x[e] = rv ? x[e] : 0.f;
         qf[s][e] = (_Float16)x[e];
         if constexpr (QLO) ql[s][e] = (_Float16)(x[e] - (float)qf[s][e]);
+      }
+#pragma unroll
+      for (int e = 0; e < 8; ++e) x[e] = fminf(fmaxf(x[e], -kLoMax), kLoMax);
+#pragma unroll
+      for (int w = 0; w < 2; ++w) {
+        const int lo2 = __builtin_amdgcn_cvt_pk_fp8_f32(x[4 * w], x[4 * w + 1], 0, false) & 0xffff;
+        const int hi2 = __builtin_amdgcn_cvt_pk_fp8_f32(x[4 * w + 2], x[4 * w + 3], 0, false) & 0xffff;
+        e8[s][w] = lo2 | (hi2 << 16);
+      }
+    }
+#pragma unroll
+    for (int c = 0; c < NLO; ++c) {
+#pragma unroll
+      for (int u = 0; u < 2; ++u) {
+#pragma unroll
+        for (int w = 0; w < 2; ++w) {
+          const auto x = __builtin_amdgcn_permlane32_swap(e8[4 * c + u][w], e8[4 * c + 2 + u][w], false, false);
+          qe[c][4 * u + w] = x[0];
+          qe[c][4 * u + 2 + w] = x[1];
+        }
       }
     }
   }
@@ -512,14 +537,46 @@ __global__ __launch_bounds__(64 * kDenseWaves) void flash_kernel(FlashArgs a) {
   const float inv = l > 0.f ? 1.f / l : 0.f;
   const long ob = (q_row0 + r / gqa) * a.o_s0 + (long)(h * gqa + r % gqa) * a.o_s1;
   if (a.lse && hh == 0) a.lse[(q_row0 + r / gqa) * a.hq + h * gqa + r % gqa] = l > 0.f ? m_run + __log2f(l) : -kInf;
+  if (a.out_dtype == ECHOKV_F32) {
+    float* op = (float*)a.out + ob + 4 * hh;
+#pragma unroll
+    for (int db = 0; db < NDB; ++db) {
+#pragma unroll
+      for (int g = 0; g < 4; ++g) {
+        float4 o;
+        o.x = acc[db][4 * g] * inv, o.y = acc[db][4 * g + 1] * inv;
+        o.z = acc[db][4 * g + 2] * inv, o.w = acc[db][4 * g + 3] * inv;
+        st_n<4>(op, ECHOKV_F32, 32 * db + 8 * g, &o.x);
+      }
+    }
+    return;
+  }
+  // 16-bit rows: the half-waves exchange their channels of two groups, so that each lane
+  // stores 16 consecutive bytes.
+  uint8_t* op = (uint8_t*)a.out + 2 * ob + 16 * hh;
+  const bool bf = a.out_dtype == ECHOKV_BF16;
 #pragma unroll
   for (int db = 0; db < NDB; ++db) {
 #pragma unroll
-    for (int g = 0; g < 4; ++g) {
-      float o[4];
+    for (int g = 0; g < 4; g += 2) {
+      uint32_t w[2][2];
 #pragma unroll
-      for (int e = 0; e < 4; ++e) o[e] = acc[db][4 * g + e] * inv;
-      st_n<4>(a.out, a.out_dtype, ob + 32 * db + 8 * g + 4 * hh, o);
+      for (int u = 0; u < 2; ++u) {
+#pragma unroll
+        for (int e = 0; e < 2; ++e) {
+          const float o0 = acc[db][4 * (g + u) + 2 * e] * inv, o1 = acc[db][4 * (g + u) + 2 * e + 1] * inv;
+          if (bf) w[u][e] = f32_to_bf16(o0) | ((uint32_t)f32_to_bf16(o1) << 16);
+          else w[u][e] = __builtin_bit_cast(uint32_t, h2_t{(_Float16)o0, (_Float16)o1});
+        }
+      }
+      u4_any_t o;
+#pragma unroll
+      for (int e = 0; e < 2; ++e) {
+        const auto x = __builtin_amdgcn_permlane32_swap(w[0][e], w[1][e], false, false);
+        o[e] = x[0];
+        o[2 + e] = x[1];
+      }
+      *(u4_any_t*)(op + 64 * db + 16 * g) = o;
     }
   }
 }

@@ -646,6 +646,38 @@ def test_fused_prefill_key_ranges_at_their_edges(device, monkeypatch, d, gqa, bs
         check(f"prefill ranges D{d} GQA{gqa} bs{bs} kg{kg} vg{vg} {str(dt)[6:]} scale {scale:.3f} cap {cap}", out, ref)
 
 
+@pytest.mark.parametrize("d,gqa,dt", [(128, 4, torch.bfloat16), (128, 7, torch.float16), (64, 8, torch.bfloat16),
+                                      (128, 4, torch.float32), (64, 5, torch.float32)])
+def test_two_pass_prefill_query_and_output_rows_of_any_alignment(device, d, gqa, dt):
+    """The flash kernel reads a query row as 16-byte words and stores 16-bit output rows by
+    16 bytes after an exchange between half-waves: chunks that leave waves without rows and
+    tiles with a few, query and output rows at odd element offsets, each output type; against
+    the oracle, the same bits as contiguous rows, and nothing written beside the rows."""
+    h, bs, kg, vg = 2, 64, 32, 32
+    lens, chunks = np.array([66, 300, 1000]), (66, 65, 257)
+    store, table = build_layer(device, lens, 4, h=h, d=d, bs=bs, kg=kg, vg=vg, dtype=dt, seed=37)
+    table_d = torch.from_numpy(table).to(device, torch.int32)
+    prefill, row = [], 2
+    for n, nq in zip(lens.tolist(), chunks):
+        prefill.append((row, row + nq, n, 0))
+        row += nq
+    reqs = list(range(len(lens)))
+    gen = torch.Generator(device=device)
+    gen.manual_seed(370)
+    wide = torch.randn(row, gqa * h, d + 3, device=device, generator=gen).to(dt)
+    q = wide[..., 3:].contiguous()
+    full = torch.zeros(row, gqa * h, d, device=device)
+    pf.prefill_attention(store, q, full, prefill, reqs, table_d, d ** -0.5)
+    ref = OA.prefill_attention(oracle_view(store), q.float().cpu().numpy(), prefill, reqs, table, d ** -0.5,
+                               vectorized=True)
+    check(f"two-pass prefill D{d} GQA{gqa} {str(dt)[6:]}", full[2:], ref[2:])
+    for odt in (torch.float32, torch.float16, torch.bfloat16):
+        buf = torch.full((row, gqa * h, d + 3), 7.0, device=device, dtype=odt)
+        pf.prefill_attention(store, wide[..., 3:], buf[..., 1 : d + 1], prefill, reqs, table_d, d ** -0.5)
+        assert torch.equal(buf[2:, :, 1 : d + 1], full[2:].to(odt))
+        assert (buf[:2] == 7).all() and (buf[..., 0] == 7).all() and (buf[..., d + 1 :] == 7).all()
+
+
 @pytest.mark.parametrize("bits", [2, 4, 8])
 def test_decode_over_a_layer_view_spanning_more_than_4_gib(device, bits):
     """One layer's view of a pool interleaved across 32 layers (page stride = 32
