@@ -385,8 +385,9 @@ __global__ __launch_bounds__(kDecThreads, GS * NO == 1 ? 4 : 2) void decode_any_
         pairs(rv.v[n], n, cat.bits, c);
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
-          // Keys past the split, and rows without a chunk, add zeros (their bytes are arbitrary).
-          const bool live = cat.ok && i < n_live;
+          // Keys past the split, rows without a chunk and blocks left out add zeros: their bytes
+          // are arbitrary, and a weight of 0 times an infinity is not 0.
+          const bool live = opened && cat.ok && i < n_live;
           const float vs = live ? (float)u2h(rv.vs[n][i])[0] : 0.f, vm = live ? (float)u2h(rv.vm[n][i])[0] : 0.f;
           float x[8];
 #pragma unroll

@@ -829,3 +829,34 @@ def test_tier_passes_at_other_shapes(device, d, gqa, qdt, ws):
     check(f"tier passes D{d} GQA{gqa} {str(qdt)[6:]}{' static' if ws else ''}", got, ref)
     alone = dec.decode_attention(store, q[3:4], table_d[3:4], lens_d[3:4], d ** -0.5, **kw)
     assert torch.equal(alone[0], got[3])
+
+
+@pytest.mark.parametrize("d,bs,kg,vg", [(96, 16, 16, 24), (160, 32, 32, 32), (100, 16, 16, 20), (128, 48, 16, 32)])
+def test_fp32_decode_leaves_out_blocks_outside_the_layer(device, d, bs, kg, vg):
+    """Block ids outside the layer (negative, or past its last page) are left out whatever
+    page 0 holds, where their reads are sent: with every byte of page 0 0xFF (fp16 NaN
+    statistics) and such ids inside, at the start and at the end of a context, the result is
+    the oracle's over the other blocks."""
+    lens = np.array([64, 97, 300, 129])
+    store, table = build_layer(device, lens, 4, h=2, d=d, bs=bs, kg=kg, vg=vg, seed=41)
+    nb = store.pages.shape[0]
+    bad = [(0, 0, -1), (1, 1, nb), (2, 2, nb + 7), (2, 3, -2), (3, -(-129 // bs) - 1, nb)]
+    bad += [(i, j, nb) for i, j in np.argwhere(table == 0).tolist()]  # nothing reads page 0 by its id
+    for i, j, v in bad:
+        table[i, j] = v
+    store.pages[0] = 0xFF
+    ps = oracle_view(store)
+    gen = torch.Generator(device=device)
+    gen.manual_seed(410)
+    q = torch.randn(len(lens), 8, d, device=device, generator=gen)
+    ref = np.zeros((len(lens), 8, d))
+    for i, n in enumerate(lens.tolist()):
+        pos = np.arange(n)
+        blk = table[i][pos // bs]
+        keep = (blk >= 0) & (blk < nb)
+        k, v = ps.gather_vec(blk[keep], pos[keep] % bs)
+        ref[i] = OA.attend(q[i].cpu().numpy(), k, v, d ** -0.5)
+    for bps in (1, 16):
+        got = dec.decode_attention(store, q, torch.from_numpy(table).to(device, torch.int32),
+                                   torch.from_numpy(lens).to(device), d ** -0.5, blocks_per_split=bps, num_splits=32)
+        check(f"left-out blocks D{d} bs{bs} bps{bps}", got, ref)
