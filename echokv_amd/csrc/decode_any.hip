@@ -99,10 +99,11 @@ __global__ __launch_bounds__(kDecThreads, GS * NO == 1 ? 4 : 2) void decode_any_
   const int g0 = a.g0 + cg * GS;
   const int gs = a.gs - cg * GS < GS ? a.gs - cg * GS : GS;
   const int qh0 = h * a.gqa + g0;
-  // Item n's channels: [ch0(n), ch0(n) + 8); a lane past the head reads octet 0 (its
-  // queries are zeros).
+  // Item n's channels: [ch0(n), ch0(n) + 8); a lane past the head reads octet 0 and scores
+  // zeros with it (not octet 0's keys times a query of 0: a key can be infinite).
   auto oct_of = [&](int n) { return l + n * GW; };
   auto ch0 = [&](int n) { return 8 * oct_of(n) < D ? 8 * oct_of(n) : 0; };
+  auto past = [&](int n) { return 8 * oct_of(n) >= D; };
 
   // ---- the chain of loads: block table, header, codes ------------------------
   // As in prefill.hip: nothing loaded is looked at before the batch that needs it,
@@ -221,7 +222,7 @@ __global__ __launch_bounds__(kDecThreads, GS * NO == 1 ? 4 : 2) void decode_any_
     const bool res = key && (unsigned long)x.rs < (unsigned long)a.res.rows && rk.rg == grp;
 #pragma unroll 1
     for (int e = 0; e < 8; ++e) {
-      const int ch = ch0(n) + e;
+      const int ch = 8 * oct_of(n) + e;  // past the head: zeros
       float v = 0.f;
       if (rb >= 0 && ch < D && res) {
         v = ld(a.res.ptr, a.res.dtype, x.rs * a.res.s0 + (long)(oo % L.KG) * a.res.s1 + (long)h * a.res.s2 + ch);
@@ -293,8 +294,8 @@ __global__ __launch_bounds__(kDecThreads, GS * NO == 1 ? 4 : 2) void decode_any_
       if constexpr (FAST) {
         h2_t c[4][4];
         pairs(rk.k[n], n, at.bits, c);
-        const uint32_t sw[4] = {rk.ks[n].x, rk.ks[n].y, rk.ks[n].z, rk.ks[n].w};
-        const uint32_t mw[4] = {rk.km[n].x, rk.km[n].y, rk.km[n].z, rk.km[n].w};
+        const uint4 ks = past(n) ? uint4{} : rk.ks[n], km = past(n) ? uint4{} : rk.km[n];
+        const uint32_t sw[4] = {ks.x, ks.y, ks.z, ks.w}, mw[4] = {km.x, km.y, km.z, km.w};
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
           float x[8];
@@ -328,6 +329,8 @@ __global__ __launch_bounds__(kDecThreads, GS * NO == 1 ? 4 : 2) void decode_any_
             float x[8];
             ld_n<8>(a.res.ptr, a.res.dtype,
                     head.rs * a.res.s0 + (long)((at.off + i) & (L.KG - 1)) * a.res.s1 + (long)h * a.res.s2 + ch0(n), x);
+#pragma unroll
+            for (int e = 0; e < 8; ++e) x[e] = past(n) ? 0.f : x[e];
             score(n, i, x);
           }
         }

@@ -860,3 +860,25 @@ def test_fp32_decode_leaves_out_blocks_outside_the_layer(device, d, bs, kg, vg):
         got = dec.decode_attention(store, q, torch.from_numpy(table).to(device, torch.int32),
                                    torch.from_numpy(lens).to(device), d ** -0.5, blocks_per_split=bps, num_splits=32)
         check(f"left-out blocks D{d} bs{bs} bps{bps}", got, ref)
+
+
+@pytest.mark.parametrize("d,gqa", [(96, 4), (40, 1), (160, 3)])
+def test_fp32_decode_with_an_infinite_key_channel(device, d, gqa):
+    """A key of the open K group (the residual, float32) with one channel at -inf scores -inf
+    for queries positive there: it has no weight, and the other keys' result stands -- also
+    in the lanes past the head, which read the head's first channels with queries of zero."""
+    lens = np.array([21, 40, 300])
+    store, table = build_layer(device, lens, 4, h=2, d=d, bs=16, kg=16, vg=8, dtype=torch.float32, seed=43)
+    rows = store.block_res[torch.from_numpy(table[np.arange(3), (lens - 1) // 16]).to(device)]
+    assert (rows >= 0).all()
+    for r in rows.tolist():
+        store.res_k[r, 2, :, 3] = -float("inf")  # position 2 of the group of every sequence's last block
+    gen = torch.Generator(device=device)
+    gen.manual_seed(430)
+    q = torch.randn(3, 2 * gqa, d, device=device, generator=gen)
+    q[..., 3] = q[..., 3].abs() + 0.1
+    ref = OA.decode_attention(oracle_view(store), q.cpu().numpy(), table, lens, d ** -0.5, vectorized=True)
+    assert np.isfinite(ref).all()
+    got = dec.decode_attention(store, q, torch.from_numpy(table).to(device, torch.int32),
+                               torch.from_numpy(lens).to(device), d ** -0.5)
+    check(f"infinite key D{d}", got, ref)
