@@ -67,9 +67,9 @@ __device__ __forceinline__ float row_sum(float x) {
 }
 
 // FAST (DecodeArgs::any_fast): power-of-two block size and K group of at least 4, whole
-// octets inside one V group, aligned rows. Other layouts are read element by element.
+// octets inside one V group, aligned rows. Other layouts read their items by item_general.
 template <int GW, int NO, int GS, bool FAST>
-__global__ __launch_bounds__(kDecThreads, GS * NO == 1 ? 4 : 2) void decode_any_kernel(DecodeArgs a) {
+__global__ __launch_bounds__(kDecThreads, FAST && GS * NO == 1 ? 4 : 2) void decode_any_kernel(DecodeArgs a) {
   constexpr int RPW = 64 / GW;     // rows per wave
   constexpr int BK = RPW * 4;      // keys per batch
   constexpr int CH = 8 * NO;       // channels per lane
@@ -214,28 +214,10 @@ __global__ __launch_bounds__(kDecThreads, GS * NO == 1 ? 4 : 2) void decode_any_
       for (int i = 0; i < 4; ++i) code_pairs<8>(w[i], sh, c[i]);
     }
   };
-  // Element by element (!FAST): channels ch0(n) .. + 7 of key off + i.
-  auto slow8 = [&](const Head& x, const At& t, int n, int i, bool live, bool key, float* y) {
-    const int oo = t.off + i, grp = oo / L.KG;
-    const long pg = page_of(x.blk) * L.stride;
-    const long rb = live ? row_base_h(L, page_of(x.blk), x.hd(), oo, t.bits) : -1;
-    const bool res = key && (unsigned long)x.rs < (unsigned long)a.res.rows && rk.rg == grp;
-#pragma unroll 1
-    for (int e = 0; e < 8; ++e) {
-      const int ch = 8 * oct_of(n) + e;  // past the head: zeros
-      float v = 0.f;
-      if (rb >= 0 && ch < D && res) {
-        v = ld(a.res.ptr, a.res.dtype, x.rs * a.res.s0 + (long)(oo % L.KG) * a.res.s1 + (long)h * a.res.s2 + ch);
-      } else if (rb >= 0 && ch < D) {
-        const long p = rb + (key ? 0 : (long)L.H * D * t.bits / 8) + (long)h * (D * t.bits / 8) + ((ch * t.bits) >> 3);
-        const float code = (float)((a.pages[p] >> ((ch * t.bits) & 7)) & ((1u << t.bits) - 1u));
-        const long st = key ? ((long)grp * L.H + h) * D + ch : ((long)oo * L.H + h) * G + ch / L.VG;
-        v = code * (float)*f16p(a.pages, pg + (key ? L.o_ks : L.o_vs) + 2 * st) +
-            (float)*f16p(a.pages, pg + (key ? L.o_km : L.o_vm) + 2 * st);
-      }
-#pragma unroll
-      for (int u = 0; u < 8; ++u) y[u] = u == e ? v : y[u];
-    }
+  // The same for the other layouts (!FAST): the item's keys or values of octet n, `live` of them.
+  auto general = [&](auto key, const Head& x, const At& t, int n, int live, float (*y)[8]) {
+    item_general<decltype(key)::value>(L, a.pages, a.res, page_of(x.blk), x.hd(), x.rs, rk.rg, t.off, t.bits, live, h,
+                                       8 * oct_of(n), y);
   };
 
   const int n_batches = (t_end - t_begin + BK - 1) / BK;
@@ -306,12 +288,10 @@ __global__ __launch_bounds__(kDecThreads, GS * NO == 1 ? 4 : 2) void decode_any_
           __builtin_amdgcn_sched_barrier(0);
         }
       } else {
+        float x[4][8];
+        general(std::true_type{}, head, at, n, opened ? n_live : 0, x);
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          float x[8] = {};
-          slow8(head, at, n, i, opened && i < n_live, true, x);
-          score(n, i, x);
-        }
+        for (int i = 0; i < 4; ++i) score(n, i, x[i]);
       }
     }
     if (FAST && __builtin_amdgcn_ballot_w64(in_res || !at.ok)) {
@@ -399,12 +379,10 @@ __global__ __launch_bounds__(kDecThreads, GS * NO == 1 ? 4 : 2) void decode_any_
           __builtin_amdgcn_sched_barrier(0);
         }
       } else {
+        float x[4][8];
+        general(std::false_type{}, cur, cat, n, opened ? n_live : 0, x);
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          float x[8] = {};
-          slow8(cur, cat, n, i, opened && i < n_live, false, x);
-          add(i, x);
-        }
+        for (int i = 0; i < 4; ++i) add(i, x[i]);
       }
     }
     if (more) load_v(at);

@@ -882,3 +882,22 @@ def test_fp32_decode_with_an_infinite_key_channel(device, d, gqa):
     got = dec.decode_attention(store, q, torch.from_numpy(table).to(device, torch.int32),
                                torch.from_numpy(lens).to(device), d ** -0.5)
     check(f"infinite key D{d}", got, ref)
+
+
+@pytest.mark.parametrize("d,bs,kg,vg", [(100, 48, 6, 20), (36, 16, 2, 1), (128, 16, 2, 2), (160, 80, 10, 5),
+                                        (64, 48, 6, 64)])
+@pytest.mark.parametrize("bits", [8, 4, 2])
+def test_fp32_decode_of_items_that_straddle_groups(device, d, bs, kg, vg, bits):
+    """Layouts whose 4-key x 8-channel items cross K groups (2 to 10 keys), V groups (1 to 5
+    channels), blocks' chunks (tokens per chunk not a power of two) or the head's end,
+    with the open group in the residual: decode equals the oracle."""
+    lens = np.array([1, 5, 47, 49, 131, 300])
+    store, table = build_layer(device, lens, bits, h=2, d=d, bs=bs, kg=kg, vg=vg, seed=47, outliers=0.02)
+    gen = torch.Generator(device=device)
+    gen.manual_seed(470)
+    for gqa in (1, 4):
+        q = torch.randn(len(lens), 2 * gqa, d, device=device, generator=gen)
+        ref = OA.decode_attention(oracle_view(store), q.cpu().numpy(), table, lens, d ** -0.5, vectorized=True)
+        got = dec.decode_attention(store, q, torch.from_numpy(table).to(device, torch.int32),
+                                   torch.from_numpy(lens).to(device), d ** -0.5, blocks_per_split=1, num_splits=8)
+        check(f"straddling items D{d} bs{bs} kg{kg} vg{vg} GQA{gqa} int{bits}", got, ref, tol=4e-4)
