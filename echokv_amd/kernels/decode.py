@@ -20,6 +20,7 @@ import torch
 from echokv_amd import _lib
 
 BLOCKS_PER_SPLIT = 16
+STATIC_BYTES = 64 << 20  # the library's static scratch
 SHORT_SPLITS = 4  # a short sequence's splits (csrc/args.h, split_blocks); fewer are not cut finer
 MAX_SPLITS = 64  # default cap: more, shorter splits keep every CU busy at small batch
 
@@ -74,7 +75,9 @@ def decode_attention(
     caller-owned ``(acc, ml)`` float32 holding ``workspace_rows(...)`` rows of ``Hq * D``
     and ``Hq * 2`` values (``S * splits`` rows at most), or ``"static"``: the
     library's static scratch (no allocation at all, for code under graph capture; at
-    most 64 MiB of workspace, and calls on one GPU must not overlap).
+    most 64 MiB of workspace, and calls on one GPU must not overlap). Without
+    ``num_splits`` the workspace does not change the result (``"static"``: as long as
+    64 MiB hold ``SHORT_SPLITS`` splits of every sequence).
     ``tier`` selects the kernel specialised for that tier; by default the tier most
     of the store's blocks are stored at. Blocks of other tiers are read correctly
     either way. With ``batch_invariant`` (the default, as the reference's decode) each
@@ -95,16 +98,18 @@ def decode_attention(
     _lib.require_device(query, block_table, seq_lens, store.pages)
     s = seq_lens.shape[0]
     hq, d = query.shape[1], query.shape[2]
-    # Short sequences are cut finer where the splits they need are there in every call: a
-    # caller's num_splits of at least SHORT_SPLITS, or the call's own count and workspace. A
-    # caller's workspace with the call's own count keeps the count it was sized for.
-    flags = _lib.DECODE_BATCH_INVARIANT if batch_invariant else 0
+    # Short sequences are cut finer by every call that has the splits for it. The call's own
+    # count is at least SHORT_SPLITS whichever workspace it uses, so that all give the same
+    # bits; a caller's workspace that holds only the splits the lengths need is left alone.
+    fewest = num_splits
     if num_splits is None:
-        num_splits = default_splits(block_table, L.block_size, blocks_per_split, max_len)
-        if batch_invariant and workspace is None:
+        fewest = num_splits = default_splits(block_table, L.block_size, blocks_per_split, max_len)
+        if batch_invariant:
             num_splits = max(num_splits, SHORT_SPLITS)
-            flags |= _lib.DECODE_SHORT_SPLITS
-    elif batch_invariant and num_splits >= SHORT_SPLITS:
+            if workspace == "static" and s * num_splits * hq * (d + 2) * 4 > STATIC_BYTES:
+                num_splits = fewest
+    flags = _lib.DECODE_BATCH_INVARIANT if batch_invariant else 0
+    if batch_invariant and num_splits >= SHORT_SPLITS:
         flags |= _lib.DECODE_SHORT_SPLITS
     if query.stride(2) != 1:
         query = query.contiguous()
@@ -124,13 +129,18 @@ def decode_attention(
         acc = ml = None
     else:
         rows = workspace_rows(store, hq, query.dtype, s, num_splits, flags)
+        if workspace is not None:
+            held = min(workspace[0].numel() // (hq * d), workspace[1].numel() // (hq * 2))
+            if held < rows and fewest < num_splits:
+                need = workspace_rows(store, hq, query.dtype, s, fewest, flags & ~_lib.DECODE_SHORT_SPLITS)
+                workspace = None if held >= need else workspace
         if workspace is None:
             acc = torch.empty(rows, hq, d, device=dev, dtype=torch.float32)
             ml = torch.empty(rows, hq, 2, device=dev, dtype=torch.float32)
+        elif held < rows:
+            raise ValueError(f"decode workspace holds fewer than the {rows} rows this call needs")
         else:
             acc, ml = workspace
-            if acc.numel() < rows * hq * d or ml.numel() < rows * hq * 2:
-                raise ValueError(f"decode workspace holds fewer than the {rows} rows this call needs")
     if isinstance(tier_mask, str):
         if tier_mask != "auto":
             raise ValueError(f"tier_mask must be an int32 device tensor or 'auto', got {tier_mask!r}")

@@ -901,3 +901,28 @@ def test_fp32_decode_of_items_that_straddle_groups(device, d, bs, kg, vg, bits):
         got = dec.decode_attention(store, q, torch.from_numpy(table).to(device, torch.int32),
                                    torch.from_numpy(lens).to(device), d ** -0.5, blocks_per_split=1, num_splits=8)
         check(f"straddling items D{d} bs{bs} kg{kg} vg{vg} GQA{gqa} int{bits}", got, ref, tol=4e-4)
+
+
+def test_decode_bits_do_not_depend_on_whose_workspace_it_is(device):
+    """A call without num_splits gives the same bits with its own workspace, a caller's (of the
+    rows of default_splits, of fewer than a short sequence's splits take, or of more) and the
+    library's static one."""
+    bs, h, gqa, d = 64, 2, 4, 128
+    lens = np.array([1, 130, 500, 1024, 1025, 1337])
+    store, table = build_layer(device, lens, 4, h=h, d=d, bs=bs, kg=32, vg=32, mem_bits=4, seed=19)
+    gen = torch.Generator(device=device)
+    gen.manual_seed(190)
+    q = torch.randn(len(lens), gqa * h, d, device=device, generator=gen).half()
+    table_d, lens_d = torch.from_numpy(table).to(device, torch.int32), torch.from_numpy(lens).to(device)
+    own = dec.decode_attention(store, q, table_d, lens_d, d ** -0.5)
+
+    def pair(rows):
+        return (torch.empty(rows, gqa * h, d, device=device), torch.empty(rows, gqa * h, 2, device=device))
+
+    n = dec.default_splits(table_d, bs, dec.BLOCKS_PER_SPLIT, None)
+    assert n < dec.SHORT_SPLITS
+    for ws in (pair(dec.workspace_rows(store, gqa * h, q.dtype, len(lens), n, 1)), pair(4 * len(lens)),
+               pair(9 * len(lens)), "static"):
+        assert torch.equal(dec.decode_attention(store, q, table_d, lens_d, d ** -0.5, workspace=ws), own)
+    with pytest.raises(ValueError, match="fewer than"):
+        dec.decode_attention(store, q, table_d, lens_d, d ** -0.5, workspace=pair(len(lens)))
