@@ -299,7 +299,8 @@ __global__ __launch_bounds__(256, QLO && D > 64 ? 1 : 2) void prefill_kernel(Pre
   // Scores are scaled inside the exponent, and the max is taken on unscaled scores,
   // which needs the scale positive: a negative one flips the query's sign (exact), a
   // zero one becomes 2^-100 (every weight equal, and masked scores stay -inf).
-  const float scale = fmaxf(fabsf(a.scale_log2), 7.8886090522101181e-31f);
+  constexpr float kTinyScale = 7.8886090522101181e-31f;
+  const float scale = fabsf(a.scale_log2) < kTinyScale ? kTinyScale : fabsf(a.scale_log2);  // NaN stays
 
   // Query fragments (B operand of S^T): row = 16*RB*wave + 16*rb + n, channels
   // 32j + 8c .. +8 in natural order.

@@ -926,3 +926,13 @@ def test_decode_bits_do_not_depend_on_whose_workspace_it_is(device):
         assert torch.equal(dec.decode_attention(store, q, table_d, lens_d, d ** -0.5, workspace=ws), own)
     with pytest.raises(ValueError, match="fewer than"):
         dec.decode_attention(store, q, table_d, lens_d, d ** -0.5, workspace=pair(len(lens)))
+
+
+def test_fused_prefill_with_a_scale_that_is_not_a_number(device):
+    """A softmax scale of NaN gives NaN, as softmax does."""
+    store, table = build_layer(device, np.array([40]), 4, h=1, seed=3)
+    q = torch.ones(5, 4, 128, device=device)
+    out = torch.zeros_like(q)
+    pf.prefill_attention(store, q, out, [(0, 5, 40, 0)], [0], torch.from_numpy(table).to(device, torch.int32),
+                         float("nan"))
+    assert out.isnan().all()
