@@ -450,17 +450,18 @@ __global__ __launch_bounds__(256, QLO && D > 64 ? 1 : 2) void prefill_kernel(Pre
           for (int j = 0; j < NPV; ++j) acc[rb][j] *= alpha;
         }
         const float m_safe = m_run[rb] == -__builtin_inff() ? 0.f : m_run[rb];
+        // The row sum takes the float32 weights: the log-sum-exp is made of it.
+        float psum[2] = {0.f, 0.f};
 #pragma unroll
         for (int kh = 0; kh < NKH; ++kh) {
 #pragma unroll
-          for (int i = 0; i < 4; ++i)
-            pb[rb][kh >> 1][4 * (kh & 1) + i] = (_Float16)__builtin_amdgcn_exp2f(__builtin_fmaf(s[rb][kh][i], scale, -m_safe));
+          for (int i = 0; i < 4; ++i) {
+            const float p = __builtin_amdgcn_exp2f(__builtin_fmaf(s[rb][kh][i], scale, -m_safe));
+            psum[i & 1] += p;
+            pb[rb][kh >> 1][4 * (kh & 1) + i] = (_Float16)p;
+          }
         }
-        // The row sum takes the fp16 weights that the PV product uses.
-        const h2_t one = {(_Float16)1.0f, (_Float16)1.0f};
-#pragma unroll
-        for (int e = 0; e < SB / 4; e += 2)
-          l_lane[rb] = __builtin_amdgcn_fdot2(h2_t{pb[rb][e >> 3][e & 7], pb[rb][e >> 3][(e & 7) + 1]}, one, l_lane[rb], false);
+        l_lane[rb] += psum[0] + psum[1];
       }
 #pragma unroll
       for (int ps = 0; ps < SB / 32; ++ps) {

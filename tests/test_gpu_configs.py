@@ -936,3 +936,37 @@ def test_fused_prefill_with_a_scale_that_is_not_a_number(device):
     pf.prefill_attention(store, q, out, [(0, 5, 40, 0)], [0], torch.from_numpy(table).to(device, torch.int32),
                          float("nan"))
     assert out.isnan().all()
+
+
+@pytest.mark.parametrize("d,vg,bs", [(128, 32, 16), (64, 32, 16), (128, 32, 48), (256, 32, 16)])
+def test_fused_prefill_sums_its_weights_in_float32(device, d, vg, bs):
+    """The row sum, and the log-sum-exp made of it, adds float32 weights: with every key but
+    one at weight 0.5 (1 + 0.9 / 1024 / 2), which fp16 rounds to 0.5 (4.4e-4 less), the
+    log-sum-exp is the float64 one. Its float32 value near 10 and the scores' 22-bit
+    operands leave about 4e-6."""
+    h, gqa, n, hot = 1, 2, 300, 37
+    layout = TieredLayout(h, d, bs, 8, 16, vg)
+    nb = -(-n // bs)
+    page = bs * TieredLayout.per_token_bytes(h, d, 8, 16, vg)
+    store = TieredKVCache(layout, torch.zeros(nb, page, dtype=torch.uint8, device=device), residual_slots=4,
+                          residual_dtype=torch.float32)
+    k = torch.zeros(n, h, d, device=device)
+    k[hot, :, 0] = 2.0
+    store.write(k, torch.randn(n, h, d, device=device), torch.arange(n, device=device), 8)
+    table = torch.arange(nb, device=device, dtype=torch.int32)[None]
+    ks, _ = oracle_view(store).gather_vec(np.arange(n) // bs, np.arange(n) % bs)
+    top = float(ks[hot, 0, 0])
+    assert (np.delete(ks[:, 0, 0], hot) == 0).all() and 1.9 < top < 2.1
+    delta = -np.log2(0.5 * (1 + 0.9 / 2048))  # the hot key's score above the others, log2 units
+    q = torch.zeros(1, gqa * h, d, device=device)
+    scale = 0.25
+    q[..., 0] = delta * np.log(2) / (top * scale)
+    out, lse = torch.zeros_like(q), torch.zeros(1, gqa * h, device=device)
+    prefill = [(0, 1, n, 0)]
+    pf.prefill_attention_fused(store, q, out, prefill, [0], table, scale, lse=lse)
+    seen = (n - 1) // 16 * 16
+    s = ks[:seen, 0, 0].astype(np.float64) * float(q[0, 0, 0]) * scale / np.log(2)
+    ref = s.max() + np.log2(np.exp2(s - s.max()).sum())
+    err = float((lse.double().cpu() - ref).abs().max())
+    print(f"[lse D{d} bs{bs}] err {err:.2e}", flush=True)
+    assert err <= 1e-5
