@@ -433,12 +433,8 @@ int prefill_run(const echokv_layout* L, const uint8_t* pages, const int64_t* blo
   a.bs_shift = __builtin_ctz((unsigned)L->block_size);
   a.kg_shift = __builtin_ctz((unsigned)L->k_group);
   a.kc_mul = chunk_mul(KC);
-  const int qa = q_dtype == ECHOKV_F32 ? 4 : 8;  // elements per 16 bytes
-  const uintptr_t oa = out_dtype == ECHOKV_F32 ? 16 : 8;
   a.fast = !(L->block_size & (L->block_size - 1)) && !(L->k_group & (L->k_group - 1)) && L->k_group >= 4 &&
-           L->v_group % 8 == 0 && KC <= 4 && L->num_blocks * KC < (1LL << 24) && (uintptr_t)pages % 16 == 0 &&
-           (uintptr_t)query % 16 == 0 && q_s0 % qa == 0 && q_s1 % qa == 0 && (uintptr_t)out % oa == 0 &&
-           o_s0 % 4 == 0 && o_s1 % 4 == 0;
+           L->v_group % 8 == 0 && KC <= 4 && L->num_blocks * KC < (1LL << 24) && (uintptr_t)pages % 16 == 0;
   if (mfma) return launched(ek::launch_prefill(a, n_tiles, (hipStream_t)stream));
   if (n_tiles > INT32_MAX / L->num_kv_heads) return ECHOKV_EINVAL;
   for (int g0 = 0; g0 < gqa; g0 += 16) {  // passes of 16 query heads per KV head

@@ -304,9 +304,8 @@ struct PrefillArgs {
   float* acc;
   float* ml;
   // 1: the MFMA kernel's items (4 keys x 8 channels) sit in one K group and V group, the
-  // block size and K group are powers of two (bs_shift, kg_shift: their logs), chunk ids
-  // are under 2^24 (page = umulhi(id, kc_mul); kc_mul 0: one chunk a page), and query /
-  // output rows are aligned for 16-byte loads / four-channel stores.
+  // block size and K group are powers of two (bs_shift, kg_shift: their logs), and chunk ids
+  // are under 2^24 (page = umulhi(id, kc_mul); kc_mul 0: one chunk a page).
   int fast, bs_shift, kg_shift;
   uint32_t kc_mul;
 };

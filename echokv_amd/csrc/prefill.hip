@@ -31,7 +31,9 @@
 // header, codes) that is spread over the steps: step i + 1's codes, step i + 2's
 // header and step i + 3's table entry are requested before step i's products.
 // Items whose keys or channels straddle a group (K group not a multiple of 4, V
-// group not of 8) are read element by element instead.
+// group not of 8), and blocks or groups that are not powers of two, are read by
+// item_general in the step that needs them (64 chunks of 16-32 tokens over 1-4K keys at
+// block 48: 1190 us element by element, 614 so).
 #include "items.h"
 
 namespace ek {
@@ -66,26 +68,30 @@ struct Raw {
   bool ok;                // the item's keys can be read
 };
 
-// Four consecutive elements by one store (aligned). DT is a template parameter so that
-// the dtype branch sits outside the caller's loop (the kernel's code is fetched cold
-// at every launch: its size is time).
+// Query and output rows: vectors at any element's alignment.
+typedef float f4_any_t __attribute__((ext_vector_type(4), aligned(4)));
+typedef _Float16 h8_any_t __attribute__((ext_vector_type(8), aligned(2)));
+typedef _Float16 h4_any_t __attribute__((ext_vector_type(4), aligned(2)));
+typedef __bf16 b4_any_t __attribute__((ext_vector_type(4), aligned(2)));
+
+// Four consecutive elements by one store. DT is a template parameter so that the dtype
+// branch sits outside the caller's loop (the kernel's code is fetched cold at every
+// launch: its size is time).
 template <int DT>
 __device__ __forceinline__ void st4v(void* p, long i, const f4_t x) {
   if constexpr (DT == ECHOKV_F32) {
-    *(f4_t*)((float*)p + i) = x;
+    *(f4_any_t*)((float*)p + i) = x;
   } else if constexpr (DT == ECHOKV_F16) {
-    *(h4_t*)((_Float16*)p + i) = h4_t{(_Float16)x[0], (_Float16)x[1], (_Float16)x[2], (_Float16)x[3]};
+    *(h4_any_t*)((_Float16*)p + i) = h4_any_t{(_Float16)x[0], (_Float16)x[1], (_Float16)x[2], (_Float16)x[3]};
   } else {
-    typedef __bf16 b4_t __attribute__((ext_vector_type(4)));
-    *(b4_t*)((__bf16*)p + i) = b4_t{(__bf16)x[0], (__bf16)x[1], (__bf16)x[2], (__bf16)x[3]};
+    *(b4_any_t*)((__bf16*)p + i) = b4_any_t{(__bf16)x[0], (__bf16)x[1], (__bf16)x[2], (__bf16)x[3]};
   }
 }
 
 }  // namespace
 
 // FAST (PrefillArgs::fast): power-of-two block size and K group, items inside one K group
-// and V group, query and output rows aligned for 16-byte loads and four-channel
-// stores. Everything else takes the same kernel with items read element by element.
+// and V group. Other layouts take the same kernel with items read by item_general.
 template <int D, bool QLO, int RB, bool FAST>
 __global__ __launch_bounds__(256, QLO && D > 64 ? 1 : 2) void prefill_kernel(PrefillArgs a) {
   constexpr int KEYS = 8192 / D;            // keys per step: 256 items of 4 keys x 8 channels
@@ -259,34 +265,15 @@ __global__ __launch_bounds__(256, QLO && D > 64 ? 1 : 2) void prefill_kernel(Pre
       }
       return;
     }
-#pragma unroll 1
-    for (int i = 0; i < 4; ++i) {
-      const int o = off + i, grp = o / L.KG;
-      const long rb = valid(step, x) ? row_base_h(L, x.blk, x.hd(), o, bits) : -1;
-      const bool live = rb >= 0 && kp + i < k_end;
-      const long hb = (long)(h * D + ch) * bits / 8;
-      const bool res = has_res && w.rg == grp;
-#pragma unroll 1
-      for (int e = 0; e < 8; ++e) {
-        float kx = 0.f, vx = 0.f;
-        if (live) {
-          const long byte = rb + hb + e * bits / 8;
-          const int sh = (e * bits) & 7;
-          const uint32_t mask = (1u << bits) - 1u;
-          const long ve = ((long)o * L.H + h) * G + (ch + e) / L.VG;
-          vx = (float)((a.pages[byte + (long)L.H * D * bits / 8] >> sh) & mask) * (float)*f16p(a.pages, pg + L.o_vs + 2 * ve) +
-               (float)*f16p(a.pages, pg + L.o_vm + 2 * ve);
-          const long se = ((long)grp * L.H + h) * D + ch + e;
-          kx = res ? ld(a.res.ptr, a.res.dtype, x.rs * a.res.s0 + (long)(o % L.KG) * a.res.s1 + h * a.res.s2 + ch + e)
-                   : (float)((a.pages[byte] >> sh) & mask) * (float)*f16p(a.pages, pg + L.o_ks + 2 * se) +
-                         (float)*f16p(a.pages, pg + L.o_km + 2 * se);
-        }
-        const int at = (key0 + i) * D + 8 * k_slot<D>(key0 + i, oct) + e;
-        kt[at] = (_Float16)kx;
-        ktl[at] = (_Float16)(kx - (float)kt[at]);
-        vt[v_at(e) + i] = (_Float16)vx;
-      }
-    }
+    const int n_live = valid(step, x) ? k_end - kp : 0;
+    float y[4][8];
+    item_general<true>(L, a.pages, a.res, page_of(x.blk), x.hd(), x.rs, w.rg, off, bits, n_live, h, ch, y);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) put_k(i, y[i]);
+    item_general<false>(L, a.pages, a.res, page_of(x.blk), x.hd(), x.rs, w.rg, off, bits, n_live, h, ch, y);
+#pragma unroll
+    for (int e = 0; e < 8; ++e)
+      *(h4_t*)&vt[v_at(e)] = h4_t{(_Float16)y[0][e], (_Float16)y[1][e], (_Float16)y[2][e], (_Float16)y[3][e]};
   };
 
   const int n_steps = (k_end - k_begin + KEYS - 1) / KEYS;
@@ -314,10 +301,10 @@ __global__ __launch_bounds__(256, QLO && D > 64 ? 1 : 2) void prefill_kernel(Pre
     qlim[rb] = og_limit(q_pos0 + tok, a.og_mask);
     const long qb = (q_row0 + tok) * a.q_s0 + (long)hh * a.q_s1;
     // Rows past the tile read its first row (never written out).
-    if constexpr (FAST && QLO) {
+    if constexpr (QLO) {
 #pragma unroll
       for (int j = 0; j < NQK; ++j) {
-        const f4_t* src = (const f4_t*)((const float*)a.q + qb + 32 * j + 8 * c);
+        const f4_any_t* src = (const f4_any_t*)((const float*)a.q + qb + 32 * j + 8 * c);
         const f4_t u = src[0], v = src[1];
 #pragma unroll
         for (int e = 0; e < 8; ++e) {
@@ -326,22 +313,12 @@ __global__ __launch_bounds__(256, QLO && D > 64 ? 1 : 2) void prefill_kernel(Pre
           qfl[rb][j][e] = (_Float16)(x - (float)qf[rb][j][e]);
         }
       }
-    } else if constexpr (FAST) {
-#pragma unroll
-      for (int j = 0; j < NQK; ++j) qf[rb][j] = *(const h8_t*)((const _Float16*)a.q + qb + 32 * j + 8 * c);
     } else {
 #pragma unroll
-      for (int j = 0; j < NQK; ++j) {
-#pragma unroll
-        for (int e = 0; e < 8; ++e) {
-          const float x = ld(a.q, a.q_dtype, qb + 32 * j + 8 * c + e);
-          qf[rb][j][e] = (_Float16)x;
-          if constexpr (QLO) qfl[rb][j][e] = (_Float16)(x - (float)qf[rb][j][e]);
-        }
-      }
+      for (int j = 0; j < NQK; ++j) qf[rb][j] = *(const h8_any_t*)((const _Float16*)a.q + qb + 32 * j + 8 * c);
     }
   }
-  if (FAST && !QLO && a.q_dtype == ECHOKV_BF16) {
+  if (!QLO && a.q_dtype == ECHOKV_BF16) {
 #pragma unroll
     for (int rb = 0; rb < RB; ++rb)
 #pragma unroll
@@ -510,18 +487,10 @@ __global__ __launch_bounds__(256, QLO && D > 64 ? 1 : 2) void prefill_kernel(Pre
       if (a.lse && c == 0)
         a.lse[row * a.hq + qh] = l_lane[rb] > 0.f ? m_run[rb] + __log2f(l_lane[rb]) : -__builtin_inff();
 #pragma unroll
-      for (int j = 0; j < NPV; ++j) {
-        if constexpr (DT >= 0) {
-          st4v<DT>(a.out, ob + 16 * j + 4 * c, acc[rb][j]);
-        } else {
-#pragma unroll
-          for (int i = 0; i < 4; ++i) st(a.out, a.out_dtype, ob + 16 * j + 4 * c + i, acc[rb][j][i]);
-        }
-      }
+      for (int j = 0; j < NPV; ++j) st4v<DT>(a.out, ob + 16 * j + 4 * c, acc[rb][j]);
     });
   };
-  if constexpr (!FAST) put_out(std::integral_constant<int, -1>{});
-  else if (a.out_dtype == ECHOKV_BF16) put_out(std::integral_constant<int, ECHOKV_BF16>{});
+  if (a.out_dtype == ECHOKV_BF16) put_out(std::integral_constant<int, ECHOKV_BF16>{});
   else if (a.out_dtype == ECHOKV_F16) put_out(std::integral_constant<int, ECHOKV_F16>{});
   else put_out(std::integral_constant<int, ECHOKV_F32>{});
 }

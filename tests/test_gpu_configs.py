@@ -600,7 +600,7 @@ def test_head_size_256_prefill_on_the_mfma_kernel(device, h, gqa, dt, bits):
     (128, 4, 64, 32, 32, torch.bfloat16, True),   # own-group part: the ranges' log-sum-exp
     (64, 7, 128, 64, 32, torch.float32, False),   # query lo part
     (256, 4, 32, 32, 32, torch.bfloat16, False),
-    (128, 1, 48, 16, 64, torch.float16, False),   # items read element by element: block size,
+    (128, 1, 48, 16, 64, torch.float16, False),   # items read by runs of channels: block size,
     (64, 4, 16, 16, 4, torch.float16, False)])    # V group
 def test_fused_prefill_key_ranges_at_their_edges(device, monkeypatch, d, gqa, bs, kg, vg, dt, og):
     """The fused kernel's key ranges (128 keys here): contexts on and around the range
@@ -970,3 +970,26 @@ def test_fused_prefill_sums_its_weights_in_float32(device, d, vg, bs):
     err = float((lse.double().cpu() - ref).abs().max())
     print(f"[lse D{d} bs{bs}] err {err:.2e}", flush=True)
     assert err <= 1e-5
+
+
+@pytest.mark.parametrize("d,bs,kg,vg,dt", [(128, 16, 2, 2, torch.float16), (64, 48, 6, 1, torch.bfloat16),
+                                           (256, 80, 10, 4, torch.float32)])
+@pytest.mark.parametrize("bits", [8, 4, 2])
+def test_fused_prefill_of_items_that_straddle_groups(device, d, bs, kg, vg, dt, bits):
+    """Such layouts on the fused prefill kernel: K groups, V groups and chunks that cross items,
+    contexts that end in an item."""
+    lens = np.array([1, 5, 47, 131, 300, 700])
+    store, table = build_layer(device, lens, bits, h=2, d=d, bs=bs, kg=kg, vg=vg, dtype=dt, seed=53, outliers=0.02)
+    prefill, row = [], 0
+    for n, nq in zip(lens.tolist(), (1, 5, 30, 64, 3, 17)):
+        prefill.append((row, row + nq, n, 0))
+        row += nq
+    gen = torch.Generator(device=device)
+    gen.manual_seed(530)
+    q = torch.randn(row, 8, d, device=device, generator=gen).to(dt)
+    out = torch.zeros(row, 8, d, device=device)
+    reqs = list(range(len(lens)))
+    pf.prefill_attention(store, q, out, prefill, reqs, torch.from_numpy(table).to(device, torch.int32), d ** -0.5)
+    ref = OA.prefill_attention(oracle_view(store), q.float().cpu().numpy(), prefill, reqs, table, d ** -0.5,
+                               vectorized=True)
+    check(f"straddling prefill items D{d} bs{bs} kg{kg} vg{vg} int{bits}", out, ref)
