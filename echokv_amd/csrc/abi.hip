@@ -381,8 +381,7 @@ int prefill_run(const echokv_layout* L, const uint8_t* pages, const int64_t* blo
                 const echokv_residual* res, const void* query, int64_t q_s0, int64_t q_s1, int32_t q_dtype,
                 int32_t num_q_heads, void* out, int64_t o_s0, int64_t o_s1, int32_t out_dtype,
                 const int32_t* tiles, int64_t n_tiles, int32_t tile_m, const int32_t* block_table, int64_t bt_s0,
-                float softmax_scale, int32_t own_group, float* lse, int32_t n_splits, int32_t split_keys,
-                int64_t part_rows, float* acc, float* ml, echokv_stream_t stream) {
+                float softmax_scale, int32_t own_group, float* lse, int32_t n_splits, int64_t part_rows, float* acc, float* ml, echokv_stream_t stream) {
   if (!lay_ok(L)) return ECHOKV_ESHAPE;
   if (num_q_heads <= 0 || num_q_heads % L->num_kv_heads) return ECHOKV_ESHAPE;
   const int gqa = num_q_heads / L->num_kv_heads;
@@ -396,7 +395,7 @@ int prefill_run(const echokv_layout* L, const uint8_t* pages, const int64_t* blo
   if (own_group && (L->k_group & (L->k_group - 1))) return ECHOKV_ESHAPE;
   if (!dtype_ok(q_dtype) || !dtype_ok(out_dtype)) return ECHOKV_EDTYPE;
   if (n_tiles < 0 || !res_ok(res)) return ECHOKV_EINVAL;
-  if (n_splits < 1 || n_splits > ek::kPrefillMaxSplits || split_keys < 1 || split_keys % 128) return ECHOKV_EINVAL;
+  if (n_splits < 1 || n_splits > ek::kPrefillMaxSplits) return ECHOKV_EINVAL;
   if (n_splits > 1 && (!mfma || !acc || !ml || part_rows < 1)) return ECHOKV_EINVAL;
   if (n_tiles == 0) return ECHOKV_OK;
   if (!pages || !block_res || !res_group || !query || !out || !tiles || !block_table) return ECHOKV_EINVAL;
@@ -425,7 +424,6 @@ int prefill_run(const echokv_layout* L, const uint8_t* pages, const int64_t* blo
   a.g0 = 0;
   a.gs = gqa;
   a.n_splits = n_splits;
-  a.split_keys = split_keys;
   a.part_rows = part_rows;
   a.acc = acc;
   a.ml = ml;
@@ -453,7 +451,7 @@ int echokv_prefill(const echokv_layout* L, const uint8_t* pages, const int64_t* 
                    const int32_t* tiles, int64_t n_tiles, int32_t tile_m, const int32_t* block_table, int64_t bt_s0,
                    float softmax_scale, int32_t own_group, float* lse, echokv_stream_t stream) {
   return prefill_run(L, pages, block_res, res_group, res, query, q_s0, q_s1, q_dtype, num_q_heads, out, o_s0, o_s1,
-                     out_dtype, tiles, n_tiles, tile_m, block_table, bt_s0, softmax_scale, own_group, lse, 1, 128, 0,
+                     out_dtype, tiles, n_tiles, tile_m, block_table, bt_s0, softmax_scale, own_group, lse, 1, 0,
                      nullptr, nullptr, stream);
 }
 
@@ -462,11 +460,10 @@ int echokv_prefill_split(const echokv_layout* L, const uint8_t* pages, const int
                          int64_t q_s1, int32_t q_dtype, int32_t num_q_heads, void* out, int64_t o_s0, int64_t o_s1,
                          int32_t out_dtype, const int32_t* tiles, int64_t n_tiles, int32_t tile_m,
                          const int32_t* block_table, int64_t bt_s0, float softmax_scale, int32_t own_group, float* lse,
-                         int32_t n_splits, int32_t split_keys, int64_t part_rows, float* acc, float* ml,
-                         echokv_stream_t stream) {
+                         int32_t n_splits, int64_t part_rows, float* acc, float* ml, echokv_stream_t stream) {
   return prefill_run(L, pages, block_res, res_group, res, query, q_s0, q_s1, q_dtype, num_q_heads, out, o_s0, o_s1,
                      out_dtype, tiles, n_tiles, tile_m, block_table, bt_s0, softmax_scale, own_group, lse, n_splits,
-                     split_keys, part_rows, acc, ml, stream);
+                     part_rows, acc, ml, stream);
 }
 
 int64_t echokv_prefill_dense_workspace(const echokv_layout* L, int64_t n_packs) {

@@ -295,11 +295,11 @@ struct PrefillArgs {
   int og_mask;  // nonzero: a query at position p sees keys < (p & og_mask) (its own K group left out)
   float* lse;   // nullable: [rows, hq] log2-domain log-sum-exp of each query row's scores
   int g0, gs;   // fp32 kernel (prefill_any): this pass's query heads of each KV head, gs <= 16
-  // MFMA kernel: a tile's context in ranges of split_keys keys (a multiple of 128), at
-  // most n_splits of them (the last takes the rest). With n_splits > 1, range z of query
-  // row r and head qh leaves its unnormalized output and (max in log2 units, sum) in row
+  // MFMA kernel: a tile's context in ranges of prefill_range(ctx) keys, at most n_splits
+  // of them (the last takes the rest). With n_splits > 1, range z of query row r and
+  // head qh leaves its unnormalized output and (max in log2 units, sum) in row
   // (z * part_rows + r) * hq + qh of acc [.., D] and ml [.., 2].
-  int n_splits, split_keys;
+  int n_splits;
   long part_rows;
   float* acc;
   float* ml;
@@ -309,7 +309,17 @@ struct PrefillArgs {
   int fast, bs_shift, kg_shift;
   uint32_t kc_mul;
 };
+// Keys per range of a context, from its own length alone: what a chunk gives must not
+// depend on the rest of the batch. 512 up to 32K keys, then the power of two that leaves
+// 64 ranges. A shorter range costs full batches (64 chunks of 16-32 tokens over 1-4K keys: 389 us
+// in one range, 414 at 512, 460 at 256; 64 chunks of 64 over 512 keys: 121 at 512, 207 at
+// 256), a longer one lone chunks (64 tokens over 8K: 67 us at 512, 105 at 1024).
 constexpr int kPrefillMaxSplits = 64;
+__host__ __device__ inline int prefill_range(int ctx) {
+  int per = 512;
+  while ((long)per * kPrefillMaxSplits < ctx) per *= 2;
+  return per;
+}
 
 struct PackArgs {
   Lay L;

@@ -16,9 +16,9 @@
 // 32-key contraction maps lane group c's eight k-slots to keys
 // {4c..4c+3, 16+4c..16+4c+3}, and V^T rows hold the keys in that order.
 //
-// Key ranges (PrefillArgs::split_keys): short chunks over long contexts give few
+// Key ranges (prefill_range): short chunks over long contexts give few
 // (tile, head) pairs, and a pair's context is a serial chain of steps. So a tile's
-// context is cut into ranges of split_keys keys, one workgroup each; a range leaves
+// context is cut into ranges by its own length, one workgroup each; a range leaves
 // its rows' unnormalized output and (max, sum), and prefill_merge_kernel adds them.
 // A tile whose context is one range writes its rows directly. 4 chunks of 5-64
 // tokens over 0.7-8K-token INT4 contexts, H 8, D 128: 850 us in one range per pair, 61 us
@@ -118,9 +118,10 @@ __global__ __launch_bounds__(256, QLO && D > 64 ? 1 : 2) void prefill_kernel(Pre
   int kv_end = q_pos0 + n_tok;
   kv_end = kv_end < ctx ? kv_end : ctx;
   const bool last = (int)blockIdx.z == a.n_splits - 1;  // the last range takes the rest
-  const int k_begin = (int)blockIdx.z * a.split_keys;
+  const int per = prefill_range(ctx);
+  const int k_begin = (int)blockIdx.z * per;
   if (blockIdx.z > 0 && k_begin >= kv_end) return;
-  const int k_end = last || kv_end - k_begin < a.split_keys ? kv_end : k_begin + a.split_keys;
+  const int k_end = last || kv_end - k_begin < per ? kv_end : k_begin + per;
 
   // ---- this thread's item of a step, and its chain of loads ----------------
   const int oct = tid % OCTS, quad = tid / OCTS;
@@ -455,7 +456,7 @@ __global__ __launch_bounds__(256, QLO && D > 64 ? 1 : 2) void prefill_kernel(Pre
     }
   }
 
-  const bool direct = a.n_splits == 1 || kv_end <= a.split_keys;  // the tile is one range
+  const bool direct = a.n_splits == 1 || kv_end <= per;  // the tile is one range
 #pragma unroll
   for (int rb = 0; rb < RB; ++rb) {
     l_lane[rb] += __shfl_xor(l_lane[rb], 16, 64);
@@ -503,14 +504,15 @@ __global__ __launch_bounds__(256) void prefill_merge_kernel(PrefillArgs a) {
   const int32_t* td = a.tiles + (long)blockIdx.x * 5;
   const int n_tok = td[1], q_pos0 = td[2], ctx = td[3];
   const int kv_end = q_pos0 + n_tok < ctx ? q_pos0 + n_tok : ctx;
-  if (kv_end <= a.split_keys) return;
+  const int range = prefill_range(ctx);
+  if (kv_end <= range) return;
   const int lane = threadIdx.x & 63;
   const int r = (int)blockIdx.z * 4 + (int)(threadIdx.x >> 6);
   if (r >= n_tok * a.gqa) return;
   const int h = blockIdx.y;
   const long row = td[0] + r / a.gqa;
   const int qh = h * a.gqa + r % a.gqa;
-  int ns = (kv_end + a.split_keys - 1) / a.split_keys;
+  int ns = (kv_end + range - 1) / range;
   ns = ns < a.n_splits ? ns : a.n_splits;  // at most 64
   const long base = row * a.hq + qh, per = a.part_rows * a.hq;
   // The (max, sum) pairs and the first 16 ranges' rows are requested together.

@@ -40,11 +40,7 @@ from echokv_amd._util import to_device
 
 ROWS = 128  # query rows (tokens x GQA heads) per workgroup of the fused kernel
 FUSED_MAX_CHUNK = 64  # the fused kernel only when every chunk is this short
-# Key ranges of the fused kernel (csrc/prefill.hip): two workgroups fit a CU.
-SPLIT_SLOTS = 512
-SPLIT_MIN_KEYS = 256
-SPLIT_STEP = 128  # ranges are whole steps of every head size's kernel
-SPLIT_MAX = 64
+RANGE_KEYS, MAX_RANGES = 512, 64  # key ranges of the fused kernel's contexts (csrc/args.h, prefill_range)
 DENSE_ROWS = 256  # query rows per workgroup of the two-pass path
 DENSE_KEYS = 64  # keys per workspace tile
 
@@ -68,21 +64,14 @@ def any_block_m(gqa: int) -> int:
     return 1 if gqa >= 16 else 16 // gqa
 
 
-def fused_splits(prefill, tile_m: int, heads: int) -> tuple[int, int]:
-    """(ranges, keys per range) of the fused kernel's contexts: every tile's context is
-    cut into ranges of one length, the shortest that leaves at most ``SPLIT_SLOTS``
-    (tile, KV head, range) triples -- one more than the chip holds at once would run
-    after all the others. A range is at least ``SPLIT_MIN_KEYS`` keys (under that a
-    workgroup's start-up and its partial rows cost more than its keys)."""
-    tiles = [(-(-(qe - qs) // tile_m), ctx) for qs, qe, ctx, *_ in prefill]
-    ctx_max = max(ctx for _, ctx in tiles)
-    slots = max(1, SPLIT_SLOTS // heads)
-    keys = sum(n * ctx for n, ctx in tiles)
-    per = max(SPLIT_MIN_KEYS, -(-keys // slots), -(-ctx_max // SPLIT_MAX))
-    per = -(-per // SPLIT_STEP) * SPLIT_STEP
-    while per < ctx_max and sum(n * -(-ctx // per) for n, ctx in tiles) > slots:
-        per += SPLIT_STEP
-    return max(1, -(-ctx_max // per)), per
+def range_keys(ctx: int) -> int:
+    """Keys per range of a ``ctx``-key context on the fused kernel, from its own length
+    alone, so that a chunk's result does not depend on the rest of the batch
+    (csrc/args.h, ``prefill_range``)."""
+    per = RANGE_KEYS
+    while per * MAX_RANGES < ctx:
+        per *= 2
+    return per
 
 
 def build_tiles(prefill, req_of, gqa: int, device, tokens: int | None = None) -> torch.Tensor:
@@ -368,9 +357,9 @@ def prefill_attention_fused(store, query: torch.Tensor, output: torch.Tensor, pr
     out = _out_view(output, hq)
     block_table = _bt(block_table)
     tiles = tiles.to(torch.int32).contiguous()
-    n_splits, split_keys, acc, ml = 1, SPLIT_STEP, None, None
+    n_splits, acc, ml = 1, None, None
     if kernels_take(L.head_size, gqa):
-        n_splits, split_keys = fused_splits(prefill, tile_m, L.num_kv_heads)
+        n_splits = max(1, max(-(-ctx // range_keys(ctx)) for _, _, ctx, *_ in prefill))
     if n_splits > 1:
         acc = torch.empty(n_splits, query.shape[0], hq, L.head_size, device=query.device, dtype=torch.float32)
         ml = torch.empty(n_splits, query.shape[0], hq, 2, device=query.device, dtype=torch.float32)
@@ -380,6 +369,6 @@ def prefill_attention_fused(store, query: torch.Tensor, output: torch.Tensor, pr
         _lib.ptr(store.res_group), _lib.byref(res), _lib.ptr(query), query.stride(0), query.stride(1),
         _lib.dtype_code(query), hq, _lib.ptr(out), out.stride(0), out.stride(1), _lib.dtype_code(out),
         _lib.ptr(tiles), tiles.shape[0], tile_m, _lib.ptr(block_table), block_table.stride(0),
-        float(softmax_scale), int(lse is not None), _lib.ptr(lse), n_splits, split_keys, query.shape[0],
+        float(softmax_scale), int(lse is not None), _lib.ptr(lse), n_splits, query.shape[0],
         _lib.ptr(acc), _lib.ptr(ml), _lib.stream(),
     )

@@ -209,10 +209,11 @@ int echokv_prefill(const echokv_layout* L, const uint8_t* pages, const int64_t* 
                    const int32_t* block_table, int64_t bt_s0, float softmax_scale,
                    int32_t own_group, float* lse, echokv_stream_t stream);
 
-/* echokv_prefill with each tile's context cut into ranges of split_keys keys (a multiple
- * of 128; at most n_splits <= 64 ranges, the last taking the rest of a longer
- * context), one workgroup per (tile, KV head, range), and a second kernel adding the
- * ranges: short chunks over long contexts then fill the chip. acc: float32
+/* echokv_prefill with each tile's context cut into ranges of 512 keys (contexts over 32768
+ * keys: the power of two that leaves 64 ranges; at most n_splits <= 64 ranges, the last
+ * taking the rest of a longer context), one workgroup per (tile, KV head, range), and a
+ * second kernel adding the ranges: short chunks over long contexts then fill the chip, and
+ * a chunk's result depends on its own request alone. acc: float32
  * [n_splits, part_rows, num_q_heads, head_size], ml: float32 [n_splits, part_rows,
  * num_q_heads, 2], part_rows > every query row of the tiles. n_splits 1: echokv_prefill
  * (acc and ml unused); more needs a layout of the MFMA kernel. Results differ from
@@ -223,7 +224,7 @@ int echokv_prefill_split(const echokv_layout* L, const uint8_t* pages, const int
                          void* out, int64_t o_s0, int64_t o_s1, int32_t out_dtype,
                          const int32_t* tiles, int64_t n_tiles, int32_t tile_m,
                          const int32_t* block_table, int64_t bt_s0, float softmax_scale,
-                         int32_t own_group, float* lse, int32_t n_splits, int32_t split_keys,
+                         int32_t own_group, float* lse, int32_t n_splits,
                          int64_t part_rows, float* acc, float* ml, echokv_stream_t stream);
 
 /* Long-chunk prefill in two passes (the dense path for chunks longer than the fused

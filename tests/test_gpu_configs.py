@@ -603,13 +603,11 @@ def test_head_size_256_prefill_on_the_mfma_kernel(device, h, gqa, dt, bits):
     (128, 1, 48, 16, 64, torch.float16, False),   # items read by runs of channels: block size,
     (64, 4, 16, 16, 4, torch.float16, False)])    # V group
 def test_fused_prefill_key_ranges_at_their_edges(device, monkeypatch, d, gqa, bs, kg, vg, dt, og):
-    """The fused kernel's key ranges (128 keys here): contexts on and around the range
+    """The fused kernel's key ranges (512 keys): contexts on and around the range
     boundaries, chunks crossing them, one-range tiles beside many-range ones, the
     range-count cap (a last range that takes the rest), a negative softmax scale and
     query rows that are not 16-byte aligned; against the oracle."""
-    monkeypatch.setattr(pf, "SPLIT_MIN_KEYS", 128)
-    monkeypatch.setattr(pf, "SPLIT_SLOTS", 1 << 20)
-    lens = np.array([1, 127, 128, 129, 255, 257, 300, 1000])
+    lens = np.array([1, 511, 512, 513, 1023, 1025, 1200, 4000])
     h = 2
     store, table = build_layer(device, lens, 4, h=h, d=d, bs=bs, kg=kg, vg=vg, dtype=dt, seed=31)
     ps = oracle_view(store)
@@ -627,10 +625,8 @@ def test_fused_prefill_key_ranges_at_their_edges(device, monkeypatch, d, gqa, bs
                           (d ** -0.5, wide[..., :d].contiguous(), 3)):
         if og and scale < 0:
             continue  # the own-group part alone takes any scale; its first part is what is tested here
-        monkeypatch.setattr(pf, "SPLIT_MAX", 64)
-        assert pf.fused_splits(prefill, pf.block_m(gqa, d), h) == (8, 128)
         if cap == 3:  # fewer ranges than the contexts need
-            monkeypatch.setattr(pf, "fused_splits", lambda *_: (3, 128))
+            monkeypatch.setattr(pf, "range_keys", lambda ctx: -(-ctx // 3))
         out = torch.zeros(row, gqa * h, d, device=device)
         kw = {}
         if og:
@@ -993,3 +989,44 @@ def test_fused_prefill_of_items_that_straddle_groups(device, d, bs, kg, vg, dt, 
     ref = OA.prefill_attention(oracle_view(store), q.float().cpu().numpy(), prefill, reqs, table, d ** -0.5,
                                vectorized=True)
     check(f"straddling prefill items D{d} bs{bs} kg{kg} vg{vg} int{bits}", out, ref)
+
+
+def test_fused_prefill_ranges_of_a_context_over_32k(device):
+    """Over 32768 keys a context's ranges are longer (1024 here): 5 tokens over 33,000 keys."""
+    n, h, gqa, d = 33000, 1, 2, 64
+    store, table = build_layer(device, np.array([n, 40]), 4, h=h, d=d, seed=59)
+    gen = torch.Generator(device=device)
+    gen.manual_seed(590)
+    q = torch.randn(8, gqa * h, d, device=device, generator=gen).half()
+    out = torch.zeros(8, gqa * h, d, device=device)
+    prefill = [(0, 5, n, 0), (5, 8, 40, 0)]
+    pf.prefill_attention(store, q, out, prefill, [0, 1], torch.from_numpy(table).to(device, torch.int32), d ** -0.5)
+    ref = OA.prefill_attention(oracle_view(store), q.float().cpu().numpy(), prefill, [0, 1], table, d ** -0.5,
+                               vectorized=True)
+    check("prefill over 33,000 keys", out, ref)
+
+
+@pytest.mark.parametrize("d,gqa,dt", [(128, 4, torch.bfloat16), (64, 4, torch.float32), (256, 4, torch.float16)])
+def test_fused_prefill_bits_do_not_depend_on_the_batch(device, d, gqa, dt):
+    """A chunk's result on the fused kernel is a function of its own request: the same bits
+    alone, with one other chunk and among many."""
+    bs, h = 64, 2
+    lens = np.array([3000, 520, 5000] + [100 + 61 * i for i in range(40)])
+    chunks = [40, 7, 64] + [1 + (13 * i) % 60 for i in range(40)]
+    store, table = build_layer(device, lens, 4, h=h, d=d, bs=bs, kg=32, vg=32, dtype=dt, seed=23)
+    table_d = torch.from_numpy(table).to(device, torch.int32)
+    gen = torch.Generator(device=device)
+    gen.manual_seed(230)
+    q = torch.randn(sum(chunks), gqa * h, d, device=device, generator=gen).to(dt)
+    o = np.concatenate([[0], np.cumsum(chunks)]).tolist()
+
+    def run(reqs):
+        out = torch.zeros_like(q)
+        pf.prefill_attention(store, q, out, [(o[i], o[i + 1], int(lens[i]), 0) for i in reqs], reqs, table_d, d ** -0.5)
+        return out
+
+    full = run(list(range(len(lens))))
+    for reqs in ([0], [1], [2], [0, 2], [1, 2], [0, 30], [1, 30, 31, 32]):
+        part = run(reqs)
+        for i in reqs:
+            assert torch.equal(part[o[i] : o[i + 1]], full[o[i] : o[i + 1]]), (reqs, i)

@@ -79,17 +79,9 @@ def test_head_size_256_tiles_hold_half_the_rows():
         pf.prefill_attention(store, q, q, prefill, req, torch.zeros(1, 1), 0.1, own_group_key=q)
 
 
-def test_fused_key_ranges_cover_the_contexts_and_fit_the_chip():
-    """Ranges cover the longest context, are whole steps, and leave at most
-    SPLIT_SLOTS (tile, head, range) triples unless a range is the whole context."""
-    cases = [[(0, 64, 8192, 0)], [(0, 1, 1, 0)], [(0, 20, 4446, 0), (20, 77, 1583, 0), (77, 111, 6215, 0)],
-             [(64 * i, 64 * i + 64, 4096 + i, 0) for i in range(40)], [(0, 3, 200000, 0)]]
-    for prefill in cases:
-        for tile_m in (1, 16, 32):
-            for heads in (1, 8):
-                n, per = pf.fused_splits(prefill, tile_m, heads)
-                ctx = max(c for _, _, c, _ in prefill)
-                assert 1 <= n <= pf.SPLIT_MAX and per % pf.SPLIT_STEP == 0 and per >= pf.SPLIT_MIN_KEYS
-                assert (n - 1) * per < ctx <= n * per or (n == 1 and ctx <= per)
-                live = sum(-(-(qe - qs) // tile_m) * -(-c // per) for qs, qe, c, _ in prefill) * heads
-                assert live <= pf.SPLIT_SLOTS or per >= ctx
+def test_fused_key_ranges_come_from_the_context_alone():
+    """Ranges are 512 keys up to 32K, then the shortest power of two that leaves 64."""
+    for ctx in (1, 511, 512, 513, 4096, 32767, 32768, 32769, 65536, 65537, 200000, 1 << 20):
+        per = pf.range_keys(ctx)
+        assert per >= 512 and per & (per - 1) == 0 and -(-ctx // per) <= pf.MAX_RANGES
+        assert per == 512 or -(-ctx // (per // 2)) > pf.MAX_RANGES
