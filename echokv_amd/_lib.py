@@ -65,7 +65,7 @@ _SIGS = {
                              P, I64, I64, I32, P],
     "echokv_prefill": [LP, P, P, P, RP, P, I64, I64, I32, I32, P, I64, I64, I32, P, I64, I32, P, I64, FL, I32, P, P],
     "echokv_prefill_split": [LP, P, P, P, RP, P, I64, I64, I32, I32, P, I64, I64, I32, P, I64, I32, P, I64, FL, I32, P,
-                             I32, I64, P, P, P],
+                             P, P, P, I64, P, P, P],
     "echokv_prefill_own_group": [LP, P, P, P, RP, P, I64, I64, I32, I32, P, I64, I64, I32, P, I64, P, I64, P, I64, I64,
                                  P, P, I64, I64, I32, FL, P],
     "echokv_prefill_dense": [LP, P, P, P, RP, P, I64, I64, I32, I32, P, I64, I64, I32, P, I64, P, I64, I32, P, I64,

@@ -381,7 +381,8 @@ int prefill_run(const echokv_layout* L, const uint8_t* pages, const int64_t* blo
                 const echokv_residual* res, const void* query, int64_t q_s0, int64_t q_s1, int32_t q_dtype,
                 int32_t num_q_heads, void* out, int64_t o_s0, int64_t o_s1, int32_t out_dtype,
                 const int32_t* tiles, int64_t n_tiles, int32_t tile_m, const int32_t* block_table, int64_t bt_s0,
-                float softmax_scale, int32_t own_group, float* lse, int32_t n_splits, int64_t part_rows, float* acc, float* ml, echokv_stream_t stream) {
+                float softmax_scale, int32_t own_group, float* lse, const int32_t* items, const int32_t* merges,
+                const int64_t* groups, int64_t n_groups, float* acc, float* ml, echokv_stream_t stream) {
   if (!lay_ok(L)) return ECHOKV_ESHAPE;
   if (num_q_heads <= 0 || num_q_heads % L->num_kv_heads) return ECHOKV_ESHAPE;
   const int gqa = num_q_heads / L->num_kv_heads;
@@ -395,8 +396,13 @@ int prefill_run(const echokv_layout* L, const uint8_t* pages, const int64_t* blo
   if (own_group && (L->k_group & (L->k_group - 1))) return ECHOKV_ESHAPE;
   if (!dtype_ok(q_dtype) || !dtype_ok(out_dtype)) return ECHOKV_EDTYPE;
   if (n_tiles < 0 || !res_ok(res)) return ECHOKV_EINVAL;
-  if (n_splits < 1 || n_splits > ek::kPrefillMaxSplits) return ECHOKV_EINVAL;
-  if (n_splits > 1 && (!mfma || !acc || !ml || part_rows < 1)) return ECHOKV_EINVAL;
+  if (n_groups < 0 || (n_groups > 0 && (!mfma || !items || !groups))) return ECHOKV_EINVAL;
+  for (int64_t i = 0; i < n_groups; ++i) {  // (first item, items, first merge, merges, first partial row) each
+    const int64_t* g = groups + 5 * i;
+    if (g[0] < 0 || g[1] < 1 || g[1] > INT32_MAX / L->num_kv_heads || g[2] < 0 || g[3] < 0 || g[3] > INT32_MAX || g[4] < 0 ||
+        (g[3] > 0 && (!merges || !acc || !ml)))
+      return ECHOKV_EINVAL;
+  }
   if (n_tiles == 0) return ECHOKV_OK;
   if (!pages || !block_res || !res_group || !query || !out || !tiles || !block_table) return ECHOKV_EINVAL;
   ek::PrefillArgs a;
@@ -423,8 +429,9 @@ int prefill_run(const echokv_layout* L, const uint8_t* pages, const int64_t* blo
   a.lse = lse;
   a.g0 = 0;
   a.gs = gqa;
-  a.n_splits = n_splits;
-  a.part_rows = part_rows;
+  a.items = nullptr;
+  a.merges = nullptr;
+  a.row0 = 0;
   a.acc = acc;
   a.ml = ml;
   const int KC = L->chunks_per_page;
@@ -433,7 +440,16 @@ int prefill_run(const echokv_layout* L, const uint8_t* pages, const int64_t* blo
   a.kc_mul = chunk_mul(KC);
   a.fast = !(L->block_size & (L->block_size - 1)) && !(L->k_group & (L->k_group - 1)) && L->k_group >= 4 &&
            L->v_group % 8 == 0 && KC <= 4 && L->num_blocks * KC < (1LL << 24) && (uintptr_t)pages % 16 == 0;
-  if (mfma) return launched(ek::launch_prefill(a, n_tiles, (hipStream_t)stream));
+  if (mfma && n_tiles > INT32_MAX / L->num_kv_heads) return ECHOKV_EINVAL;
+  if (mfma && n_groups == 0) return launched(ek::launch_prefill(a, n_tiles, 0, (hipStream_t)stream));
+  for (int64_t i = 0; i < n_groups; ++i) {  // one after the other: they share the partial rows
+    const int64_t* g = groups + 5 * i;
+    a.items = items + 4 * g[0];
+    a.merges = merges + 4 * g[2];
+    a.row0 = g[4];
+    if (ek::launch_prefill(a, g[1], g[3], (hipStream_t)stream) != hipSuccess) return ECHOKV_ELAUNCH;
+  }
+  if (mfma) return ECHOKV_OK;
   if (n_tiles > INT32_MAX / L->num_kv_heads) return ECHOKV_EINVAL;
   for (int g0 = 0; g0 < gqa; g0 += 16) {  // passes of 16 query heads per KV head
     a.g0 = g0;
@@ -451,8 +467,8 @@ int echokv_prefill(const echokv_layout* L, const uint8_t* pages, const int64_t* 
                    const int32_t* tiles, int64_t n_tiles, int32_t tile_m, const int32_t* block_table, int64_t bt_s0,
                    float softmax_scale, int32_t own_group, float* lse, echokv_stream_t stream) {
   return prefill_run(L, pages, block_res, res_group, res, query, q_s0, q_s1, q_dtype, num_q_heads, out, o_s0, o_s1,
-                     out_dtype, tiles, n_tiles, tile_m, block_table, bt_s0, softmax_scale, own_group, lse, 1, 0,
-                     nullptr, nullptr, stream);
+                     out_dtype, tiles, n_tiles, tile_m, block_table, bt_s0, softmax_scale, own_group, lse,
+                     nullptr, nullptr, nullptr, 0, nullptr, nullptr, stream);
 }
 
 int echokv_prefill_split(const echokv_layout* L, const uint8_t* pages, const int64_t* block_res,
@@ -460,10 +476,11 @@ int echokv_prefill_split(const echokv_layout* L, const uint8_t* pages, const int
                          int64_t q_s1, int32_t q_dtype, int32_t num_q_heads, void* out, int64_t o_s0, int64_t o_s1,
                          int32_t out_dtype, const int32_t* tiles, int64_t n_tiles, int32_t tile_m,
                          const int32_t* block_table, int64_t bt_s0, float softmax_scale, int32_t own_group, float* lse,
-                         int32_t n_splits, int64_t part_rows, float* acc, float* ml, echokv_stream_t stream) {
+                         const int32_t* items, const int32_t* merges, const int64_t* groups, int64_t n_groups,
+                         float* acc, float* ml, echokv_stream_t stream) {
   return prefill_run(L, pages, block_res, res_group, res, query, q_s0, q_s1, q_dtype, num_q_heads, out, o_s0, o_s1,
-                     out_dtype, tiles, n_tiles, tile_m, block_table, bt_s0, softmax_scale, own_group, lse, n_splits,
-                     part_rows, acc, ml, stream);
+                     out_dtype, tiles, n_tiles, tile_m, block_table, bt_s0, softmax_scale, own_group, lse, items,
+                     merges, groups, n_groups, acc, ml, stream);
 }
 
 int64_t echokv_prefill_dense_workspace(const echokv_layout* L, int64_t n_packs) {

@@ -68,6 +68,13 @@ struct Raw {
   bool ok;                // the item's keys can be read
 };
 
+// Ranges of a tile of n_rows query rows over kv_end keys, of the `ranges` of `rows` query
+// rows that it has partial rows for (0 or 1: it is taken in one piece).
+__device__ __forceinline__ int tile_ranges(int ranges, int rows, int n_rows, int kv_end, int per) {
+  const int need = (kv_end + per - 1) / per;
+  return n_rows > rows ? 1 : (need < ranges ? need : ranges);
+}
+
 // Query and output rows: vectors at any element's alignment.
 typedef float f4_any_t __attribute__((ext_vector_type(4), aligned(4)));
 typedef _Float16 h8_any_t __attribute__((ext_vector_type(8), aligned(2)));
@@ -105,8 +112,20 @@ __global__ __launch_bounds__(256, QLO && D > 64 ? 1 : 2) void prefill_kernel(Pre
   __shared__ __attribute__((aligned(16))) _Float16 vt[D * KEYS];
 
   const Lay& L = a.L;
-  const int tile = blockIdx.x;
-  const int h = blockIdx.y;
+  // Heads fastest: a request's tiles of one range and head are H workgroups apart, which
+  // for 8 heads is the same XCD and its L2 (4 chunks over 0.7-8K keys 69 -> 65.5 us).
+  const int h = blockIdx.x % a.L.H;
+  int tile = blockIdx.x / a.L.H, z = 0, ranges = 1;
+  long part0 = 0;  // the tile's partial rows: first, and rows per range
+  int part_rows = 0;
+  if (a.items) {
+    const int32_t* it = a.items + 4 * (long)tile;
+    tile = it[0] / kPrefillMaxRanges;
+    z = it[0] % kPrefillMaxRanges;
+    ranges = it[1];
+    part0 = it[2] - a.row0;
+    part_rows = it[3];
+  }
   const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
   const int c = lane >> 4, n = lane & 15;
   const int32_t* td = a.tiles + tile * 5;
@@ -117,11 +136,11 @@ __global__ __launch_bounds__(256, QLO && D > 64 ? 1 : 2) void prefill_kernel(Pre
   const int n_rows = n_tok * gqa;
   int kv_end = q_pos0 + n_tok;
   kv_end = kv_end < ctx ? kv_end : ctx;
-  const bool last = (int)blockIdx.z == a.n_splits - 1;  // the last range takes the rest
-  const int per = prefill_range(ctx);
-  const int k_begin = (int)blockIdx.z * per;
-  if (blockIdx.z > 0 && k_begin >= kv_end) return;
-  const int k_end = last || kv_end - k_begin < per ? kv_end : k_begin + per;
+  const int per = prefill_range(ctx, D);
+  ranges = tile_ranges(ranges, part_rows, n_rows, kv_end, per);
+  if (z > 0 && z >= ranges) return;
+  const int k_begin = z * per;
+  const int k_end = z >= ranges - 1 ? kv_end : k_begin + per;  // the last takes the rest
 
   // ---- this thread's item of a step, and its chain of loads ----------------
   const int oct = tid % OCTS, quad = tid / OCTS;
@@ -456,7 +475,7 @@ __global__ __launch_bounds__(256, QLO && D > 64 ? 1 : 2) void prefill_kernel(Pre
     }
   }
 
-  const bool direct = a.n_splits == 1 || kv_end <= per;  // the tile is one range
+  const bool direct = ranges <= 1;
 #pragma unroll
   for (int rb = 0; rb < RB; ++rb) {
     l_lane[rb] += __shfl_xor(l_lane[rb], 16, 64);
@@ -469,12 +488,12 @@ __global__ __launch_bounds__(256, QLO && D > 64 ? 1 : 2) void prefill_kernel(Pre
 #pragma unroll
     for (int rb = 0; rb < RB; ++rb) {
       const int r = 16 * RB * wave + 16 * rb + n;
-      if (r < n_rows) put(rb, q_row0 + r / gqa, h * gqa + r % gqa);
+      if (r < n_rows) put(rb, r);
     }
   };
   if (!direct) {
-    rows([&](int rb, long row, int qh) {
-      const long pr = ((long)blockIdx.z * a.part_rows + row) * a.hq + qh;
+    rows([&](int rb, int r) {
+      const long pr = (part0 + (long)z * part_rows + r) * L.H + h;
       if (c == 0) *(float2*)(a.ml + 2 * pr) = float2{m_run[rb], l_lane[rb]};
 #pragma unroll
       for (int j = 0; j < NPV; ++j) *(f4_t*)(a.acc + pr * D + 16 * j + 4 * c) = acc[rb][j];
@@ -483,7 +502,9 @@ __global__ __launch_bounds__(256, QLO && D > 64 ? 1 : 2) void prefill_kernel(Pre
   }
   auto put_out = [&](auto dt) {
     constexpr int DT = decltype(dt)::value;
-    rows([&](int rb, long row, int qh) {
+    rows([&](int rb, int r) {
+      const long row = q_row0 + r / gqa;
+      const int qh = h * gqa + r % gqa;
       const long ob = row * a.o_s0 + (long)qh * a.o_s1;
       if (a.lse && c == 0)
         a.lse[row * a.hq + qh] = l_lane[rb] > 0.f ? m_run[rb] + __log2f(l_lane[rb]) : -__builtin_inff();
@@ -497,24 +518,23 @@ __global__ __launch_bounds__(256, QLO && D > 64 ? 1 : 2) void prefill_kernel(Pre
 }
 
 // The ranges of a tile's rows added (log-sum-exp, in range order) and normalized: one
-// wave per row, lane l channels [D/64 l, D/64 (l + 1)). Rows of one-range tiles are done.
+// wave per row, lane l channels [D/64 l, D/64 (l + 1)).
 template <int D>
 __global__ __launch_bounds__(256) void prefill_merge_kernel(PrefillArgs a) {
   constexpr int C = D / 64;
-  const int32_t* td = a.tiles + (long)blockIdx.x * 5;
+  const int32_t* it = a.merges + 4 * (long)blockIdx.x;
+  const int32_t* td = a.tiles + (long)(it[0] / kPrefillMaxRanges) * 5;
   const int n_tok = td[1], q_pos0 = td[2], ctx = td[3];
   const int kv_end = q_pos0 + n_tok < ctx ? q_pos0 + n_tok : ctx;
-  const int range = prefill_range(ctx);
-  if (kv_end <= range) return;
+  const int ns = tile_ranges(it[1], it[3], n_tok * a.gqa, kv_end, prefill_range(ctx, D));  // at most 64
+  if (ns <= 1) return;  // written directly
   const int lane = threadIdx.x & 63;
   const int r = (int)blockIdx.z * 4 + (int)(threadIdx.x >> 6);
   if (r >= n_tok * a.gqa) return;
   const int h = blockIdx.y;
   const long row = td[0] + r / a.gqa;
   const int qh = h * a.gqa + r % a.gqa;
-  int ns = (kv_end + range - 1) / range;
-  ns = ns < a.n_splits ? ns : a.n_splits;  // at most 64
-  const long base = row * a.hq + qh, per = a.part_rows * a.hq;
+  const long base = (it[2] - a.row0 + r) * (long)a.L.H + h, per = (long)it[3] * a.L.H;
   // The (max, sum) pairs and the first 16 ranges' rows are requested together.
   const float2 p = lane < ns ? *(const float2*)(a.ml + 2 * (base + lane * per)) : float2{-__builtin_inff(), 0.f};
   float o[C] = {}, mm = 0.f, w = 0.f, den = 0.f;
@@ -547,29 +567,29 @@ __global__ __launch_bounds__(256) void prefill_merge_kernel(PrefillArgs a) {
   const float inv = den > 0.f ? 1.f / den : 0.f;
 #pragma unroll
   for (int e = 0; e < C; ++e) o[e] *= inv;
-  if (a.lse && lane == 0) a.lse[base] = den > 0.f ? mm + __log2f(den) : -__builtin_inff();
+  if (a.lse && lane == 0) a.lse[row * a.hq + qh] = den > 0.f ? mm + __log2f(den) : -__builtin_inff();
   st_n<C>(a.out, a.out_dtype, row * a.o_s0 + (long)qh * a.o_s1 + C * lane, o);
 }
 
 template <int D, int RB>
-static hipError_t prefill_d(const PrefillArgs& a, long n_tiles, hipStream_t s) {
-  const dim3 grid((unsigned)n_tiles, (unsigned)a.L.H, (unsigned)a.n_splits);
+static hipError_t prefill_d(const PrefillArgs& a, long n, long n_merges, hipStream_t s) {
+  const dim3 grid((unsigned)(n * a.L.H));
   const bool f32 = a.q_dtype == ECHOKV_F32;
   if (f32 && a.fast) hipLaunchKernelGGL((prefill_kernel<D, true, RB, true>), grid, dim3(256), 0, s, a);
   else if (f32) hipLaunchKernelGGL((prefill_kernel<D, true, RB, false>), grid, dim3(256), 0, s, a);
   else if (a.fast) hipLaunchKernelGGL((prefill_kernel<D, false, RB, true>), grid, dim3(256), 0, s, a);
   else hipLaunchKernelGGL((prefill_kernel<D, false, RB, false>), grid, dim3(256), 0, s, a);
   const hipError_t e = hipGetLastError();
-  if (e != hipSuccess || a.n_splits == 1) return e;
+  if (e != hipSuccess || n_merges == 0) return e;
   const unsigned rows = (unsigned)prefill_rows(D);
-  hipLaunchKernelGGL((prefill_merge_kernel<D>), dim3((unsigned)n_tiles, (unsigned)a.L.H, rows / 4), dim3(256), 0, s, a);
+  hipLaunchKernelGGL((prefill_merge_kernel<D>), dim3((unsigned)n_merges, (unsigned)a.L.H, rows / 4), dim3(256), 0, s, a);
   return hipGetLastError();
 }
 
-hipError_t launch_prefill(const PrefillArgs& a, long n_tiles, hipStream_t s) {
-  if (a.L.D == 128) return prefill_d<128, 2>(a, n_tiles, s);
-  if (a.L.D == 64) return prefill_d<64, 2>(a, n_tiles, s);
-  if (a.L.D == 256) return prefill_d<256, 1>(a, n_tiles, s);
+hipError_t launch_prefill(const PrefillArgs& a, long n, long n_merges, hipStream_t s) {
+  if (a.L.D == 128) return prefill_d<128, 2>(a, n, n_merges, s);
+  if (a.L.D == 64) return prefill_d<64, 2>(a, n, n_merges, s);
+  if (a.L.D == 256) return prefill_d<256, 1>(a, n, n_merges, s);
   return hipErrorInvalidValue;
 }
 

@@ -10,8 +10,10 @@ limit: query ``i`` of an ``nq``-token chunk over ``ctx`` keys sees keys
 Two paths, chosen as the reference chooses (``FUSED_MAX_CHUNK``,
 prefill.py:74): when every chunk is at most 64 tokens, one fused HIP kernel
 (``echokv_amd/csrc/prefill.hip``): each workgroup takes a tile of
-``128 // GQA`` query tokens of one request for one KV head, dequantizes each
-32-key tile of the context into LDS (fp16) and runs QK^T and PV on MFMA.
+``128 // GQA`` query tokens of one request, one KV head and one range of the context,
+dequantizes ``8192 // D`` keys at a time into LDS (fp16) and runs QK^T and PV on MFMA; a
+second kernel adds the ranges (``RangePlan``). The ranges come from the request's own
+context, so a chunk's result on this path does not depend on the rest of the batch.
 Longer chunks take the two-pass path (``echokv_amd/csrc/prefill_dense.hip``,
 the reference's dense dequantization + flash attention, prefill.py:133-167):
 every 64-key tile of each context is dequantized once into a workspace, then
@@ -33,6 +35,7 @@ from __future__ import annotations
 
 from typing import NamedTuple
 
+import numpy as np
 import torch
 
 from echokv_amd import _lib
@@ -41,6 +44,10 @@ from echokv_amd._util import to_device
 ROWS = 128  # query rows (tokens x GQA heads) per workgroup of the fused kernel
 FUSED_MAX_CHUNK = 64  # the fused kernel only when every chunk is this short
 RANGE_KEYS, MAX_RANGES = 512, 64  # key ranges of the fused kernel's contexts (csrc/args.h, prefill_range)
+# Float32 partial rows of the ranges that run together; a step with more runs its tiles in
+# several launches over the same rows, each with a tail of its own: 64 chunks of 16-32 tokens
+# over 1-4K keys take 394 us at 64 MiB, 374 at 128 and 337 at 256 (a single launch).
+PARTIAL_BYTES = 128 << 20
 DENSE_ROWS = 256  # query rows per workgroup of the two-pass path
 DENSE_KEYS = 64  # keys per workspace tile
 
@@ -64,14 +71,49 @@ def any_block_m(gqa: int) -> int:
     return 1 if gqa >= 16 else 16 // gqa
 
 
-def range_keys(ctx: int) -> int:
-    """Keys per range of a ``ctx``-key context on the fused kernel, from its own length
+def range_keys(ctx: np.ndarray, head_size: int = 128) -> np.ndarray:
+    """Keys per range of ``ctx``-key contexts on the fused kernel, from their own lengths
     alone, so that a chunk's result does not depend on the rest of the batch
     (csrc/args.h, ``prefill_range``)."""
-    per = RANGE_KEYS
-    while per * MAX_RANGES < ctx:
-        per *= 2
+    per = np.full_like(ctx, RANGE_KEYS * (2 if head_size == 256 else 1))
+    while (per * MAX_RANGES < ctx).any():
+        per = np.where(per * MAX_RANGES < ctx, 2 * per, per)
     return per
+
+
+class RangePlan:
+    """The key ranges of a tile table (``echokv_prefill_split``): ``items`` and ``merges`` on
+    the device, and how they split into groups that share partial rows."""
+
+    def __init__(self, tiles: np.ndarray, gqa: int, head_size: int):
+        self.head_size = head_size
+        n_tok, pos0, ctx = (tiles[:, i].astype(np.int64) for i in (1, 2, 3))
+        keys = np.minimum(pos0 + n_tok, ctx)
+        n = np.maximum(1, -(-keys // range_keys(np.maximum(ctx, 1), head_size)))
+        rows = n_tok * gqa
+        self.n_items = np.concatenate([[0], np.cumsum(n)])
+        self.n_rows = np.concatenate([[0], np.cumsum(np.where(n > 1, n * rows, 0))])
+        self.n_merges = np.concatenate([[0], np.cumsum(n > 1)])
+        tile = np.repeat(np.arange(len(n)), n)
+        z = np.arange(len(tile)) - np.repeat(self.n_items[:-1], n)
+        self.host_items = np.stack([tile * MAX_RANGES + z, n[tile], self.n_rows[tile], rows[tile]], 1).astype(np.int32)
+        self.host_merges = self.host_items[(z == 0) & (n[tile] > 1)]
+        self.items = self.merges = None
+        self._groups: dict = {}
+
+    def groups(self, limit: int) -> tuple[torch.Tensor, int]:
+        """(host table [groups, 5], partial rows of the largest group): runs of tiles with at
+        most ``limit`` partial rows together (or one tile)."""
+        if limit not in self._groups:
+            out, most, t, end = [], 0, 0, len(self.n_items) - 1
+            while t < end:
+                u = max(t + 1, int(np.searchsorted(self.n_rows, self.n_rows[t] + limit, "right")) - 1)
+                at = [(c[t], c[u] - c[t]) for c in (self.n_items, self.n_merges, self.n_rows)]
+                out.append([*at[0], *at[1], at[2][0]])
+                most = max(most, int(at[2][1]))
+                t = u
+            self._groups[limit] = torch.tensor(np.array(out, np.int64)), most
+        return self._groups[limit]
 
 
 def build_tiles(prefill, req_of, gqa: int, device, tokens: int | None = None) -> torch.Tensor:
@@ -87,8 +129,21 @@ def build_tiles(prefill, req_of, gqa: int, device, tokens: int | None = None) ->
         pos0 = ctx - nq
         for t0 in range(0, nq, bm):
             rows.append((qs + t0, min(bm, nq - t0), pos0 + t0, ctx, r))
-    tiles = to_device(torch.tensor(rows, dtype=torch.int32).reshape(-1, 5), device)
+    # Tiles of at most 64 rows are head size 256's.
+    head_size = 256 if bm * gqa <= ROWS // 2 else 128
+    return _upload_tiles(np.array(rows, np.int32).reshape(-1, 5), gqa, head_size, bm, device)
+
+
+def _upload_tiles(rows: np.ndarray, gqa: int, head_size: int, bm: int, device) -> torch.Tensor:
+    """The tile table on the device in one copy with its key ranges, both planned once per
+    step: the table carries them to every layer's call."""
+    plan = RangePlan(rows, gqa, head_size)
+    parts = [rows.ravel(), plan.host_items.ravel(), plan.host_merges.ravel()]
+    dev = to_device(torch.from_numpy(np.concatenate(parts)), device).split([p.size for p in parts])
+    tiles = dev[0].view(-1, 5)
+    plan.items, plan.merges = dev[1:]
     tiles.tile_tokens = bm  # checked against the kernel's tile size at launch, without a device read
+    tiles.ranges = plan
     return tiles
 
 
@@ -356,19 +411,23 @@ def prefill_attention_fused(store, query: torch.Tensor, output: torch.Tensor, pr
         query = query.contiguous()
     out = _out_view(output, hq)
     block_table = _bt(block_table)
+    plan = getattr(tiles, "ranges", None)
+    if kernels_take(L.head_size, gqa) and (plan is None or (plan.head_size == 256) != (L.head_size == 256)):
+        # Not from build_tiles, or of small tiles: planned from what it holds (a device sync).
+        tiles = _upload_tiles(tiles.cpu().to(torch.int32).numpy(), gqa, L.head_size, tile_m, query.device)
+    plan, ranges = getattr(tiles, "ranges", None), (None, None, None, 0, None, None)
     tiles = tiles.to(torch.int32).contiguous()
-    n_splits, acc, ml = 1, None, None
-    if kernels_take(L.head_size, gqa):
-        n_splits = max(1, max(-(-ctx // range_keys(ctx)) for _, _, ctx, *_ in prefill))
-    if n_splits > 1:
-        acc = torch.empty(n_splits, query.shape[0], hq, L.head_size, device=query.device, dtype=torch.float32)
-        ml = torch.empty(n_splits, query.shape[0], hq, 2, device=query.device, dtype=torch.float32)
+    if kernels_take(L.head_size, gqa) and plan.n_merges[-1] > 0:
+        h, d = L.num_kv_heads, L.head_size
+        groups, most = plan.groups(max(1, PARTIAL_BYTES // (h * (d + 2) * 4)))
+        partial = torch.empty(most * h * (d + 2), device=query.device, dtype=torch.float32)
+        acc, ml = partial[: most * h * d], partial[most * h * d :]
+        ranges = (*map(_lib.ptr, (plan.items, plan.merges, groups)), groups.shape[0], _lib.ptr(acc), _lib.ptr(ml))
     res = _lib.residual(store.res_k)
     _lib.call(
         "echokv_prefill_split", _lib.byref(store.abi), _lib.ptr(store.pages), _lib.ptr(store.block_res),
         _lib.ptr(store.res_group), _lib.byref(res), _lib.ptr(query), query.stride(0), query.stride(1),
         _lib.dtype_code(query), hq, _lib.ptr(out), out.stride(0), out.stride(1), _lib.dtype_code(out),
         _lib.ptr(tiles), tiles.shape[0], tile_m, _lib.ptr(block_table), block_table.stride(0),
-        float(softmax_scale), int(lse is not None), _lib.ptr(lse), n_splits, query.shape[0],
-        _lib.ptr(acc), _lib.ptr(ml), _lib.stream(),
+        float(softmax_scale), int(lse is not None), _lib.ptr(lse), *ranges, _lib.stream(),
     )

@@ -603,7 +603,7 @@ def test_head_size_256_prefill_on_the_mfma_kernel(device, h, gqa, dt, bits):
     (128, 1, 48, 16, 64, torch.float16, False),   # items read by runs of channels: block size,
     (64, 4, 16, 16, 4, torch.float16, False)])    # V group
 def test_fused_prefill_key_ranges_at_their_edges(device, monkeypatch, d, gqa, bs, kg, vg, dt, og):
-    """The fused kernel's key ranges (512 keys): contexts on and around the range
+    """The fused kernel's key ranges (512 keys, 1024 at head size 256): contexts on and around the range
     boundaries, chunks crossing them, one-range tiles beside many-range ones, the
     range-count cap (a last range that takes the rest), a negative softmax scale and
     query rows that are not 16-byte aligned; against the oracle."""
@@ -626,7 +626,7 @@ def test_fused_prefill_key_ranges_at_their_edges(device, monkeypatch, d, gqa, bs
         if og and scale < 0:
             continue  # the own-group part alone takes any scale; its first part is what is tested here
         if cap == 3:  # fewer ranges than the contexts need
-            monkeypatch.setattr(pf, "range_keys", lambda ctx: -(-ctx // 3))
+            monkeypatch.setattr(pf, "range_keys", lambda ctx, _: -(-ctx // 3))
         out = torch.zeros(row, gqa * h, d, device=device)
         kw = {}
         if og:
@@ -1030,3 +1030,49 @@ def test_fused_prefill_bits_do_not_depend_on_the_batch(device, d, gqa, dt):
         part = run(reqs)
         for i in reqs:
             assert torch.equal(part[o[i] : o[i + 1]], full[o[i] : o[i + 1]]), (reqs, i)
+
+
+@pytest.mark.parametrize("d", [128, 256])
+def test_fused_prefill_partial_rows_are_bounded_and_its_plan_is_safe(device, monkeypatch, d):
+    """A step whose ranges need more partial rows than PARTIAL_BYTES runs in groups over the
+    same rows, with the same bits; a table without a plan (a copy) gives them too; a tile
+    table that changes under its plan (longer and shorter contexts, more query rows than
+    it had partial rows for) is attended whole."""
+    h, gqa = 2, 4
+    lens = np.array([2000, 700, 513, 3000, 100, 1500])
+    chunks = [33, 64, 20, 7, 64, 40]
+    store, table = build_layer(device, lens, 4, h=h, d=d, seed=61)
+    table_d = torch.from_numpy(table).to(device, torch.int32)
+    o = np.concatenate([[0], np.cumsum(chunks)]).tolist()
+    prefill = [(o[i], o[i + 1], int(n), 0) for i, n in enumerate(lens)]
+    reqs = list(range(len(lens)))
+    gen = torch.Generator(device=device)
+    gen.manual_seed(610)
+    q = torch.randn(o[-1], gqa * h, d, device=device, generator=gen).half()
+
+    def run(tiles=None, entries=prefill):
+        out = torch.zeros(q.shape, device=device)
+        torch.cuda.reset_peak_memory_stats()
+        before = torch.cuda.memory_allocated()
+        pf.prefill_attention(store, q, out, entries, reqs, table_d, d ** -0.5, tiles=tiles)
+        return out, torch.cuda.max_memory_allocated() - before
+
+    full, used = run()
+    ref = OA.prefill_attention(oracle_view(store), q.float().cpu().numpy(), prefill, reqs, table, d ** -0.5,
+                               vectorized=True)
+    check(f"prefill groups D{d}", full, ref)
+    tiles = pf.build_tiles(prefill, reqs, gqa, device, tokens=pf.block_m(gqa, d))
+    assert torch.equal(run(tiles)[0], full) and torch.equal(run(tiles.clone())[0], full)
+    monkeypatch.setattr(pf, "PARTIAL_BYTES", 1 << 20)
+    some, less = run()
+    assert torch.equal(some, full) and less < used and less < 2 << 20
+    # The plan of shorter contexts and chunks under this step's table, and of longer ones.
+    for other in ([(a, b, b - a + 3, 0) for a, b, _, _ in prefill], [(a, a + 1 + (b - a) // 3, n, 0) for a, b, n, _ in prefill],
+                  [(a, b, 5000, 0) for a, b, _, _ in prefill]):
+        stale = pf.build_tiles(other, reqs, gqa, device, tokens=pf.block_m(gqa, d))
+        if stale.shape != tiles.shape:  # a chunk of fewer tiles: the plan alone, for as many tiles
+            rows = tiles.cpu().numpy().copy()
+            rows[:, 1] = np.maximum(1, rows[:, 1] // 3)
+            stale = pf._upload_tiles(rows, gqa, d, pf.block_m(gqa, d), device)
+        stale.copy_(tiles)
+        check(f"prefill under a stale plan D{d}", run(stale)[0], ref)

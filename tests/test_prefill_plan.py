@@ -2,6 +2,8 @@
 the two-pass path's workspace and query tiles cover every query row and every
 context key exactly once (echokv_vllm/kernels/prefill.py:56-87)."""
 
+import numpy as np
+
 from echokv_amd.kernels import prefill as pf
 
 
@@ -80,8 +82,67 @@ def test_head_size_256_tiles_hold_half_the_rows():
 
 
 def test_fused_key_ranges_come_from_the_context_alone():
-    """Ranges are 512 keys up to 32K, then the shortest power of two that leaves 64."""
-    for ctx in (1, 511, 512, 513, 4096, 32767, 32768, 32769, 65536, 65537, 200000, 1 << 20):
-        per = pf.range_keys(ctx)
-        assert per >= 512 and per & (per - 1) == 0 and -(-ctx // per) <= pf.MAX_RANGES
-        assert per == 512 or -(-ctx // (per // 2)) > pf.MAX_RANGES
+    """Ranges are 512 keys (head size 256: 1024) up to 64 of them, then the shortest power of
+    two that leaves 64."""
+    ctx = np.array([1, 511, 512, 513, 4096, 32767, 32768, 32769, 65536, 65537, 200000, 1 << 20])
+    for d, least in ((64, 512), (128, 512), (256, 1024)):
+        per = pf.range_keys(ctx, d)
+        assert (per >= least).all() and (per & (per - 1) == 0).all() and (-(-ctx // per) <= pf.MAX_RANGES).all()
+        assert ((per == least) | (-(-ctx // (per // 2)) > pf.MAX_RANGES)).all()
+
+
+def test_fused_range_plan_covers_every_tile_within_its_rows():
+    """Every tile's keys are covered once by its items, in order; its partial rows are its own
+    within its group, and a group's fit the limit unless it is one tile. The largest
+    step's partial rows stay within PARTIAL_BYTES: 60 chunks of 64 tokens beside one over 32K keys
+    took 1.0 GB when every query row had room for the most ranges."""
+    rng = np.random.default_rng(5)
+    steps = [[(0, 64, 8192, 0)], [(0, 1, 1, 0)], [(64 * i, 64 * i + 64, 64 if i else 32768, 0) for i in range(61)],
+             [(512 * i, 512 * i + 512, 4096, 0) for i in range(16)], [(0, 3, 200000, 0), (3, 10, 513, 0)],
+             [(40 * i, 40 * i + int(rng.integers(1, 40)), int(rng.integers(40, 5000)), 0) for i in range(50)]]
+    for prefill in steps:
+        for gqa, heads, d in ((4, 8, 128), (8, 1, 128), (1, 32, 64), (4, 8, 256)):
+            tiles = pf.build_tiles(prefill, list(range(len(prefill))), gqa, "cpu", tokens=pf.block_m(gqa, d))
+            plan = tiles.ranges
+            items, merges = plan.items.view(-1, 4).tolist(), plan.merges.view(-1, 4).tolist()
+            want = []
+            for t, (_, n, p0, ctx, _) in enumerate(tiles.tolist()):
+                per, keys = int(pf.range_keys(np.array([ctx]), d)[0]), min(p0 + n, ctx)
+                want += [(t, z, -(-keys // per), n * gqa) for z in range(-(-keys // per))]
+            assert [(i // 64, i % 64, n, r) for i, n, _, r in items] == want
+            assert merges == [it for it in items if it[0] % 64 == 0 and it[1] > 1]
+            for limit in (1, 1000, pf.PARTIAL_BYTES // (heads * (d + 2) * 4)):
+                groups, most = plan.groups(limit)
+                g = groups.tolist()
+                assert [sum(x[1] for x in g[:i]) for i in range(len(g) + 1)] == [x[0] for x in g] + [len(items)]
+                assert [sum(x[3] for x in g[:i]) for i in range(len(g) + 1)] == [x[2] for x in g] + [len(merges)]
+                for i0, n, m0, nm, row0 in g:
+                    used, at = 0, row0
+                    assert merges[m0 : m0 + nm] == [it for it in items[i0 : i0 + n] if it[0] % 64 == 0 and it[1] > 1]
+                    for _, ranges, first, rows in merges[m0 : m0 + nm]:
+                        assert first == at
+                        at += ranges * rows
+                    used = at - row0
+                    assert used <= most and (used <= limit or nm == 1)
+            if len(prefill) > 2:
+                assert most * heads * (d + 2) * 4 <= pf.PARTIAL_BYTES
+
+
+def test_fused_prefill_plans_its_ranges_once(monkeypatch):
+    """A table from build_tiles carries its ranges: a layer's call plans nothing."""
+    import pytest
+    import torch
+    from types import SimpleNamespace
+
+    store = SimpleNamespace(layout=SimpleNamespace(num_kv_heads=2, head_size=128), pages=torch.zeros(1))
+    prefill = [(0, 40, 4000, 0)]
+    tiles = pf.build_tiles(prefill, [0], 4, "cpu")
+
+    def plan(*_):
+        raise AssertionError("planned again")
+
+    monkeypatch.setattr(pf, "RangePlan", plan)
+    monkeypatch.setattr(pf._lib, "require_device", lambda *_: None)
+    q = torch.zeros(40, 8, 128)
+    with pytest.raises(AttributeError, match="res_k"):  # past the planning, at the store's buffers
+        pf.prefill_attention_fused(store, q, q, prefill, [0], torch.zeros(1, 1, dtype=torch.int32), 0.1, tiles)
