@@ -120,9 +120,9 @@ int echokv_write_step(const echokv_layout* L, uint8_t* pages, const void* key, i
   if (parts > 0 && fin_grid > INT32_MAX / parts) return ECHOKV_EINVAL;
   const int staged =
       vec && (parts > 0 || ek::step_staged_lds(KG, kv_dtype) <= ek::kStepStagedMaxLds) ? kv_dtype : -1;
-  // From kWideRows rows on the step is two launches of kernels made for throughput.
+  // From wide_rows rows on the step is two launches of kernels made for throughput.
   const int vl = L->v_group / 16, va = kv_dtype == ECHOKV_F32 ? 4 : 8;
-  const int wide = n_rows >= ek::kWideRows && (fin_grid == 0 || parts > 0) && L->head_size % 16 == 0 &&
+  const int wide = n_rows >= ek::wide_rows(L->num_kv_heads * L->head_size, KG) && (fin_grid == 0 || parts > 0) && L->head_size % 16 == 0 &&
                    L->v_group % 16 == 0 && !(vl & (vl - 1)) && (uintptr_t)value % 16 == 0 && v_s0 % va == 0 &&
                    v_s1 % va == 0 && (uintptr_t)pages % 16 == 0;
   ek::StepArgs a{ek::WriteTokArgs{to_lay(L), pages, key, k_s0, k_s1, value, v_s0, v_s1, kv_dtype, tok, tok_s0,

@@ -76,9 +76,17 @@ struct StepArgs {
   int wide;
 };
 
-// Token rows from which a step is two launches: both take 15 us at 1500 rows (INT4, H 8, D 128;
-// 1000: 11.0 fused, 13.9 apart; 2100: 19.2 fused, 16.2 apart; 8400: 68, 31).
-constexpr int kWideRows = 1536;
+// Token rows from which a step is two launches. Apart, the work per row is less, but two
+// kernels one after the other take 17-20 us however small the rows are, and the fin rows of
+// a K group of 64 (16 positions a thread) 2-3 us more; the fused step grows with
+// rows x channels. us fused / apart (bf16, INT4), by channels H x D and K group:
+//   1540 rows: 64/32 18.1 / 17.5, 1024/32 19.8 / 19.0, 1024/16 21.0 / 18.0, 4096/64 42.6 / 37.4;
+//              128/64 17.2 / 19.7, 1024/64 19.6 / 22.3, 2048/64 26.0 / 26.8
+//   1800 rows: 128/64 18.3 / 20.1, 1024/64 21.5 / 22.2, 2048/64 28.1 / 27.4
+//   2310 rows: 128/64 21.1 / 20.6, 256/64 20.9 / 21.1, 1024/64 24.6 / 23.4
+inline int wide_rows(int channels, int k_group) {
+  return k_group <= 32 || channels >= 4096 ? 1536 : (channels >= 2048 ? 1792 : 2304);
+}
 // Dynamic LDS of a staged fused step, and the largest the launch takes without
 // raising the kernel's limit.
 inline size_t step_staged_lds(int k_group, int dtype) {
