@@ -444,8 +444,8 @@ int prefill_run(const echokv_layout* L, const uint8_t* pages, const int64_t* blo
   if (mfma && n_groups == 0) return launched(ek::launch_prefill(a, n_tiles, 0, (hipStream_t)stream));
   for (int64_t i = 0; i < n_groups; ++i) {  // one after the other: they share the partial rows
     const int64_t* g = groups + 5 * i;
-    a.items = items + 4 * g[0];
-    a.merges = merges + 4 * g[2];
+    a.items = items + 5 * g[0];
+    a.merges = merges + 5 * g[2];
     a.row0 = g[4];
     if (ek::launch_prefill(a, g[1], g[3], (hipStream_t)stream) != hipSuccess) return ECHOKV_ELAUNCH;
   }

@@ -303,14 +303,14 @@ struct PrefillArgs {
   int og_mask;  // nonzero: a query at position p sees keys < (p & og_mask) (its own K group left out)
   float* lse;   // nullable: [rows, hq] log2-domain log-sum-exp of each query row's scores
   int g0, gs;   // fp32 kernel (prefill_any): this pass's query heads of each KV head, gs <= 16
-  // MFMA kernel: a tile's context in ranges of prefill_range keys. items: null (every
-  // tile in one range), or a row (tile * 64 + range z, the tile's ranges, its first partial
-  // row, its query rows) per workgroup and KV head; merges: the same rows for z = 0 of the
-  // tiles with more than one range. A tile whose context needs more ranges than that
-  // gives the last one the rest; one with more query rows than that is taken in one range (the
-  // tile table may have changed since). Range z of the tile's row r and KV head h leaves its
-  // unnormalized output and (max in log2 units, sum) in row
-  // (first - row0 + z * rows + r) * H + h of acc [.., D] and ml [.., 2].
+  // MFMA kernel: a tile's context in ranges of keys. items: null (every tile in one range), or
+  // a row (tile * 64 + range z, the tile's ranges, keys per range, its first partial row, its
+  // query rows) per workgroup and KV head; merges: the same rows for z = 0 of the tiles with more
+  // than one range. A tile whose context needs more ranges than that gives the last one the
+  // rest; one with more query rows than that is taken in one range (the tile table may have
+  // changed since). Range z of the tile's row r and KV head h leaves its unnormalized output and
+  // (max in log2 units, sum) in row (first - row0 + z * rows) * H + h * rows + r of acc [.., D]
+  // and ml [.., 2].
   const int32_t* items;
   const int32_t* merges;
   long row0;
@@ -322,17 +322,7 @@ struct PrefillArgs {
   int fast, bs_shift, kg_shift;
   uint32_t kc_mul;
 };
-// Keys per range of a context, from its own length alone: what a chunk gives must not
-// depend on the rest of the batch. 512 (head size 256, whose tiles are half as long and
-// their partial rows twice: 1024) up to 64 ranges, then the power of two that leaves 64. A shorter range costs full batches (64 chunks of 16-32 tokens over 1-4K keys: 389 us
-// in one range, 414 at 512, 460 at 256; 64 chunks of 64 over 512 keys: 121 at 512, 207 at
-// 256), a longer one lone chunks (64 tokens over 8K: 67 us at 512, 105 at 1024).
 constexpr int kPrefillMaxRanges = 64;
-__host__ __device__ inline int prefill_range(int ctx, int head_size) {
-  int per = head_size == 256 ? 1024 : 512;
-  while ((long)per * kPrefillMaxRanges < ctx) per *= 2;
-  return per;
-}
 
 struct PackArgs {
   Lay L;

@@ -16,9 +16,9 @@
 // 32-key contraction maps lane group c's eight k-slots to keys
 // {4c..4c+3, 16+4c..16+4c+3}, and V^T rows hold the keys in that order.
 //
-// Key ranges (prefill_range): short chunks over long contexts give few
+// Key ranges (PrefillArgs::items): short chunks over long contexts give few
 // (tile, head) pairs, and a pair's context is a serial chain of steps. So a tile's
-// context is cut into ranges by its own length, one workgroup each; a range leaves
+// context is cut into ranges, one workgroup each; a range leaves
 // its rows' unnormalized output and (max, sum), and prefill_merge_kernel adds them.
 // A tile whose context is one range writes its rows directly. 4 chunks of 5-64
 // tokens over 0.7-8K-token INT4 contexts, H 8, D 128: 850 us in one range per pair, 61 us
@@ -68,11 +68,12 @@ struct Raw {
   bool ok;                // the item's keys can be read
 };
 
-// Ranges of a tile of n_rows query rows over kv_end keys, of the `ranges` of `rows` query
-// rows that it has partial rows for (0 or 1: it is taken in one piece).
+// Ranges of `per` keys of a tile of n_rows query rows over kv_end keys, of the `ranges` of
+// `rows` query rows that it has partial rows for (0 or 1: it is taken in one piece).
 __device__ __forceinline__ int tile_ranges(int ranges, int rows, int n_rows, int kv_end, int per) {
+  if (ranges <= 1 || n_rows > rows) return 1;
   const int need = (kv_end + per - 1) / per;
-  return n_rows > rows ? 1 : (need < ranges ? need : ranges);
+  return need < ranges ? need : ranges;
 }
 
 // Query and output rows: vectors at any element's alignment.
@@ -117,14 +118,15 @@ __global__ __launch_bounds__(256, QLO && D > 64 ? 1 : 2) void prefill_kernel(Pre
   const int h = blockIdx.x % a.L.H;
   int tile = blockIdx.x / a.L.H, z = 0, ranges = 1;
   long part0 = 0;  // the tile's partial rows: first, and rows per range
-  int part_rows = 0;
+  int part_rows = 0, per = 0;
   if (a.items) {
-    const int32_t* it = a.items + 4 * (long)tile;
+    const int32_t* it = a.items + 5 * (long)tile;
     tile = it[0] / kPrefillMaxRanges;
     z = it[0] % kPrefillMaxRanges;
     ranges = it[1];
-    part0 = it[2] - a.row0;
-    part_rows = it[3];
+    per = it[2];
+    part0 = it[3] - a.row0;
+    part_rows = it[4];
   }
   const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
   const int c = lane >> 4, n = lane & 15;
@@ -136,7 +138,6 @@ __global__ __launch_bounds__(256, QLO && D > 64 ? 1 : 2) void prefill_kernel(Pre
   const int n_rows = n_tok * gqa;
   int kv_end = q_pos0 + n_tok;
   kv_end = kv_end < ctx ? kv_end : ctx;
-  const int per = prefill_range(ctx, D);
   ranges = tile_ranges(ranges, part_rows, n_rows, kv_end, per);
   if (z > 0 && z >= ranges) return;
   const int k_begin = z * per;
@@ -493,7 +494,7 @@ __global__ __launch_bounds__(256, QLO && D > 64 ? 1 : 2) void prefill_kernel(Pre
   };
   if (!direct) {
     rows([&](int rb, int r) {
-      const long pr = (part0 + (long)z * part_rows + r) * L.H + h;
+      const long pr = (part0 + (long)z * part_rows) * L.H + (long)h * part_rows + r;
       if (c == 0) *(float2*)(a.ml + 2 * pr) = float2{m_run[rb], l_lane[rb]};
 #pragma unroll
       for (int j = 0; j < NPV; ++j) *(f4_t*)(a.acc + pr * D + 16 * j + 4 * c) = acc[rb][j];
@@ -522,11 +523,11 @@ __global__ __launch_bounds__(256, QLO && D > 64 ? 1 : 2) void prefill_kernel(Pre
 template <int D>
 __global__ __launch_bounds__(256) void prefill_merge_kernel(PrefillArgs a) {
   constexpr int C = D / 64;
-  const int32_t* it = a.merges + 4 * (long)blockIdx.x;
+  const int32_t* it = a.merges + 5 * (long)blockIdx.x;
   const int32_t* td = a.tiles + (long)(it[0] / kPrefillMaxRanges) * 5;
   const int n_tok = td[1], q_pos0 = td[2], ctx = td[3];
   const int kv_end = q_pos0 + n_tok < ctx ? q_pos0 + n_tok : ctx;
-  const int ns = tile_ranges(it[1], it[3], n_tok * a.gqa, kv_end, prefill_range(ctx, D));  // at most 64
+  const int ns = tile_ranges(it[1], it[4], n_tok * a.gqa, kv_end, it[2]);  // at most 64
   if (ns <= 1) return;  // written directly
   const int lane = threadIdx.x & 63;
   const int r = (int)blockIdx.z * 4 + (int)(threadIdx.x >> 6);
@@ -534,7 +535,8 @@ __global__ __launch_bounds__(256) void prefill_merge_kernel(PrefillArgs a) {
   const int h = blockIdx.y;
   const long row = td[0] + r / a.gqa;
   const int qh = h * a.gqa + r % a.gqa;
-  const long base = (it[2] - a.row0 + r) * (long)a.L.H + h, per = (long)it[3] * a.L.H;
+  const int rows = it[4];
+  const long base = (long)(it[3] - a.row0) * a.L.H + (long)h * rows + r, per = (long)rows * a.L.H;
   // The (max, sum) pairs and the first 16 ranges' rows are requested together.
   const float2 p = lane < ns ? *(const float2*)(a.ml + 2 * (base + lane * per)) : float2{-__builtin_inff(), 0.f};
   float o[C] = {}, mm = 0.f, w = 0.f, den = 0.f;

@@ -43,10 +43,13 @@ from echokv_amd._util import to_device
 
 ROWS = 128  # query rows (tokens x GQA heads) per workgroup of the fused kernel
 FUSED_MAX_CHUNK = 64  # the fused kernel only when every chunk is this short
-RANGE_KEYS, MAX_RANGES = 512, 64  # key ranges of the fused kernel's contexts (csrc/args.h, prefill_range)
+# Key ranges of the fused kernel's contexts (range_keys): a tile's most, a request's most, and
+# a request's most of 256 keys.
+MAX_RANGES, MANY_RANGES, FEW_RANGES = 64, 64, 32
 # Float32 partial rows of the ranges that run together; a step with more runs its tiles in
 # several launches over the same rows, each with a tail of its own: 64 chunks of 16-32 tokens
-# over 1-4K keys take 394 us at 64 MiB, 374 at 128 and 337 at 256 (a single launch).
+# over 1-4K keys in ranges of 512 take 394 us at 64 MiB, 374 at 128 and 337 at 256 (a single
+# launch).
 PARTIAL_BYTES = 128 << 20
 DENSE_ROWS = 256  # query rows per workgroup of the two-pass path
 DENSE_KEYS = 64  # keys per workspace tile
@@ -71,13 +74,21 @@ def any_block_m(gqa: int) -> int:
     return 1 if gqa >= 16 else 16 // gqa
 
 
-def range_keys(ctx: np.ndarray, head_size: int = 128) -> np.ndarray:
-    """Keys per range of ``ctx``-key contexts on the fused kernel, from their own lengths
-    alone, so that a chunk's result does not depend on the rest of the batch
-    (csrc/args.h, ``prefill_range``)."""
-    per = np.full_like(ctx, RANGE_KEYS * (2 if head_size == 256 else 1))
-    while (per * MAX_RANGES < ctx).any():
-        per = np.where(per * MAX_RANGES < ctx, 2 * per, per)
+def range_keys(tiles: int, ctx: int) -> int:
+    """Keys per range of the fused kernel for a request whose chunk has ``tiles`` tiles over
+    ``ctx`` keys: from the request alone, so that its result does not depend on the rest of
+    the batch (it does on how the request is cut into chunks).
+
+    At 8 KV heads 64 ranges are a workgroup for every place the chip has, so a request is cut
+    into at most that many; 256 keys each while that leaves half the places to others (1 tile
+    over 1000 keys: 28 us at 256, 47 at 512; 2 over 4096: 40, 55; but 2 requests of 2 over 8192: 86,
+    74). A full batch pays for partial rows that one range per tile does without (64 chunks
+    of 64 tokens over 1024 keys 209 -> 342 us; over 1-4K keys 350 -> 354)."""
+    if ctx <= 512:
+        return 512
+    per = 256 if tiles * -(-ctx // 256) <= FEW_RANGES else 512
+    while 256 < per < ctx and tiles * -(-ctx // per) > MANY_RANGES:  # at most MAX_RANGES with one tile
+        per *= 2
     return per
 
 
@@ -85,19 +96,22 @@ class RangePlan:
     """The key ranges of a tile table (``echokv_prefill_split``): ``items`` and ``merges`` on
     the device, and how they split into groups that share partial rows."""
 
-    def __init__(self, tiles: np.ndarray, gqa: int, head_size: int):
-        self.head_size = head_size
-        n_tok, pos0, ctx = (tiles[:, i].astype(np.int64) for i in (1, 2, 3))
-        keys = np.minimum(pos0 + n_tok, ctx)
-        n = np.maximum(1, -(-keys // range_keys(np.maximum(ctx, 1), head_size)))
+    def __init__(self, tiles: np.ndarray, gqa: int):
+        n_tok, pos0, ctx, req = (tiles[:, i].astype(np.int64) for i in (1, 2, 3, 4))
+        new = np.ones(len(tiles), bool)  # a request's tiles are neighbours
+        new[1:] = (req[1:] != req[:-1]) | (ctx[1:] != ctx[:-1])
+        of = np.cumsum(new) - 1
+        size = np.bincount(of).tolist() if len(tiles) else []
+        per = np.array([range_keys(n, c) for n, c in zip(size, ctx[new].tolist())], np.int64)[of]
+        n = np.maximum(1, -(-np.minimum(pos0 + n_tok, ctx) // per))
         rows = n_tok * gqa
         self.n_items = np.concatenate([[0], np.cumsum(n)])
         self.n_rows = np.concatenate([[0], np.cumsum(np.where(n > 1, n * rows, 0))])
         self.n_merges = np.concatenate([[0], np.cumsum(n > 1)])
-        tile = np.repeat(np.arange(len(n)), n)
-        z = np.arange(len(tile)) - np.repeat(self.n_items[:-1], n)
-        self.host_items = np.stack([tile * MAX_RANGES + z, n[tile], self.n_rows[tile], rows[tile]], 1).astype(np.int32)
-        self.host_merges = self.host_items[(z == 0) & (n[tile] > 1)]
+        t = np.repeat(np.arange(len(n)), n)
+        z = np.arange(len(t)) - np.repeat(self.n_items[:-1], n)
+        items = np.stack([t * MAX_RANGES + z, n[t], per[t], self.n_rows[t], rows[t]], 1).astype(np.int32)
+        self.host_items, self.host_merges = items, items[(z == 0) & (n[t] > 1)]
         self.items = self.merges = None
         self._groups: dict = {}
 
@@ -129,15 +143,13 @@ def build_tiles(prefill, req_of, gqa: int, device, tokens: int | None = None) ->
         pos0 = ctx - nq
         for t0 in range(0, nq, bm):
             rows.append((qs + t0, min(bm, nq - t0), pos0 + t0, ctx, r))
-    # Tiles of at most 64 rows are head size 256's.
-    head_size = 256 if bm * gqa <= ROWS // 2 else 128
-    return _upload_tiles(np.array(rows, np.int32).reshape(-1, 5), gqa, head_size, bm, device)
+    return _upload_tiles(np.array(rows, np.int32).reshape(-1, 5), gqa, bm, device)
 
 
-def _upload_tiles(rows: np.ndarray, gqa: int, head_size: int, bm: int, device) -> torch.Tensor:
+def _upload_tiles(rows: np.ndarray, gqa: int, bm: int, device) -> torch.Tensor:
     """The tile table on the device in one copy with its key ranges, both planned once per
     step: the table carries them to every layer's call."""
-    plan = RangePlan(rows, gqa, head_size)
+    plan = RangePlan(rows, gqa)
     parts = [rows.ravel(), plan.host_items.ravel(), plan.host_merges.ravel()]
     dev = to_device(torch.from_numpy(np.concatenate(parts)), device).split([p.size for p in parts])
     tiles = dev[0].view(-1, 5)
@@ -411,10 +423,9 @@ def prefill_attention_fused(store, query: torch.Tensor, output: torch.Tensor, pr
         query = query.contiguous()
     out = _out_view(output, hq)
     block_table = _bt(block_table)
-    plan = getattr(tiles, "ranges", None)
-    if kernels_take(L.head_size, gqa) and (plan is None or (plan.head_size == 256) != (L.head_size == 256)):
-        # Not from build_tiles, or of small tiles: planned from what it holds (a device sync).
-        tiles = _upload_tiles(tiles.cpu().to(torch.int32).numpy(), gqa, L.head_size, tile_m, query.device)
+    if kernels_take(L.head_size, gqa) and getattr(tiles, "ranges", None) is None:
+        # Not from build_tiles: planned from what the table holds (a device sync).
+        tiles = _upload_tiles(tiles.cpu().to(torch.int32).numpy(), gqa, tile_m, query.device)
     plan, ranges = getattr(tiles, "ranges", None), (None, None, None, 0, None, None)
     tiles = tiles.to(torch.int32).contiguous()
     if kernels_take(L.head_size, gqa) and plan.n_merges[-1] > 0:

@@ -209,22 +209,23 @@ int echokv_prefill(const echokv_layout* L, const uint8_t* pages, const int64_t* 
                    const int32_t* block_table, int64_t bt_s0, float softmax_scale,
                    int32_t own_group, float* lse, echokv_stream_t stream);
 
-/* echokv_prefill with each tile's context cut into ranges of 512 keys (head size 256: 1024;
- * contexts of more than 64 such ranges: the power of two that leaves 64), one workgroup per (tile, KV head, range),
- * and a second kernel adding a tile's ranges: short chunks over long contexts then fill
- * the chip, and a chunk's result depends on its own request alone. The caller plans it:
- * items (device int32 [.., 4]) = (tile * 64 + range, the tile's ranges, its first partial
- * row, its query rows n_tokens * GQA) for every range of every tile (keys up to
- * min(q_pos0 + n_tokens, ctx)), a tile's one after the other; merges (device int32 [.., 4])
+/* echokv_prefill with each tile's context cut into at most 64 ranges of keys, one workgroup
+ * per (tile, KV head, range), and a second kernel adding a tile's ranges: short chunks over
+ * long contexts then fill the chip. The caller plans it: items (device int32 [.., 5]) =
+ * (tile * 64 + range, the tile's ranges, keys per range (a multiple of 128), its first
+ * partial row, its query rows n_tokens * GQA) for every range of every tile (keys up to
+ * min(q_pos0 + n_tokens, ctx)), a tile's one after the other; merges (device int32 [.., 5])
  * = those rows with range 0 of the tiles with more than one; groups (host int64
  * [n_groups, 5]) = (first item, items, first merge, merges, first partial row). Groups run
  * one after the other over the same acc [rows * num_kv_heads, head_size] and ml
  * [rows * num_kv_heads, 2] (float32), rows = the largest group's partial rows: a tile has
  * ranges * rows of them, one with a single range has none and is written directly. A tile
  * table that changed under a plan is safe: contexts that grew give the last range the rest,
- * tiles with more query rows are taken in one piece. n_groups 0: echokv_prefill (the others
- * unused); more needs a layout of the MFMA kernel. Results differ from echokv_prefill's by
- * float rounding. No counterpart in the reference. */
+ * tiles with more query rows are taken in one piece. A row's result depends on its tile's
+ * range length alone: plan that from the request, not from the batch, for results that do not
+ * depend on the batch. n_groups 0: echokv_prefill (the others unused); more needs a layout of
+ * the MFMA kernel. Results differ from echokv_prefill's by float rounding. No counterpart in
+ * the reference. */
 int echokv_prefill_split(const echokv_layout* L, const uint8_t* pages, const int64_t* block_res,
                          const int64_t* res_group, const echokv_residual* res,
                          const void* query, int64_t q_s0, int64_t q_s1, int32_t q_dtype, int32_t num_q_heads,

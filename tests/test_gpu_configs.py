@@ -603,7 +603,7 @@ def test_head_size_256_prefill_on_the_mfma_kernel(device, h, gqa, dt, bits):
     (128, 1, 48, 16, 64, torch.float16, False),   # items read by runs of channels: block size,
     (64, 4, 16, 16, 4, torch.float16, False)])    # V group
 def test_fused_prefill_key_ranges_at_their_edges(device, monkeypatch, d, gqa, bs, kg, vg, dt, og):
-    """The fused kernel's key ranges (512 keys, 1024 at head size 256): contexts on and around the range
+    """The fused kernel's key ranges (512 keys here): contexts on and around the range
     boundaries, chunks crossing them, one-range tiles beside many-range ones, the
     range-count cap (a last range that takes the rest), a negative softmax scale and
     query rows that are not 16-byte aligned; against the oracle."""
@@ -625,14 +625,17 @@ def test_fused_prefill_key_ranges_at_their_edges(device, monkeypatch, d, gqa, bs
                           (d ** -0.5, wide[..., :d].contiguous(), 3)):
         if og and scale < 0:
             continue  # the own-group part alone takes any scale; its first part is what is tested here
-        if cap == 3:  # fewer ranges than the contexts need
-            monkeypatch.setattr(pf, "range_keys", lambda ctx, _: -(-ctx // 3))
+        monkeypatch.setattr(pf, "range_keys", lambda *_: 512)
+        tiles = pf.build_tiles(prefill, reqs, gqa, device, tokens=pf.block_m(gqa, d))
+        if cap == 3:  # fewer ranges than the contexts need: the plan of shorter ones
+            tiles = pf.build_tiles([(a, b, min(n, 1400), 0) for a, b, n, _ in prefill], reqs, gqa, device,
+                                   tokens=pf.block_m(gqa, d)).copy_(tiles)
         out = torch.zeros(row, gqa * h, d, device=device)
         kw = {}
         if og:
             key = torch.randn(row, h, d, device=device, generator=gen).to(dt)
             kw = {"own_group_key": key}
-        pf.prefill_attention(store, q, out, prefill, reqs, table_d, scale, **kw)
+        pf.prefill_attention(store, q, out, prefill, reqs, table_d, scale, tiles=tiles, **kw)
         torch.cuda.synchronize()
         qn = q.float().cpu().numpy()
         if og:
@@ -992,7 +995,8 @@ def test_fused_prefill_of_items_that_straddle_groups(device, d, bs, kg, vg, dt, 
 
 
 def test_fused_prefill_ranges_of_a_context_over_32k(device):
-    """Over 32768 keys a context's ranges are longer (1024 here): 5 tokens over 33,000 keys."""
+    """Over 32768 keys a context's ranges are longer than 512 (64 ranges at most): 5 tokens over
+    33,000 keys."""
     n, h, gqa, d = 33000, 1, 2, 64
     store, table = build_layer(device, np.array([n, 40]), 4, h=h, d=d, seed=59)
     gen = torch.Generator(device=device)
@@ -1073,6 +1077,6 @@ def test_fused_prefill_partial_rows_are_bounded_and_its_plan_is_safe(device, mon
         if stale.shape != tiles.shape:  # a chunk of fewer tiles: the plan alone, for as many tiles
             rows = tiles.cpu().numpy().copy()
             rows[:, 1] = np.maximum(1, rows[:, 1] // 3)
-            stale = pf._upload_tiles(rows, gqa, d, pf.block_m(gqa, d), device)
+            stale = pf._upload_tiles(rows, gqa, pf.block_m(gqa, d), device)
         stale.copy_(tiles)
         check(f"prefill under a stale plan D{d}", run(stale)[0], ref)

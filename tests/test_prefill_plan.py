@@ -81,14 +81,21 @@ def test_head_size_256_tiles_hold_half_the_rows():
         pf.prefill_attention(store, q, q, prefill, req, torch.zeros(1, 1), 0.1, own_group_key=q)
 
 
-def test_fused_key_ranges_come_from_the_context_alone():
-    """Ranges are 512 keys (head size 256: 1024) up to 64 of them, then the shortest power of
-    two that leaves 64."""
-    ctx = np.array([1, 511, 512, 513, 4096, 32767, 32768, 32769, 65536, 65537, 200000, 1 << 20])
-    for d, least in ((64, 512), (128, 512), (256, 1024)):
-        per = pf.range_keys(ctx, d)
-        assert (per >= least).all() and (per & (per - 1) == 0).all() and (-(-ctx // per) <= pf.MAX_RANGES).all()
-        assert ((per == least) | (-(-ctx // (per // 2)) > pf.MAX_RANGES)).all()
+def test_fused_key_ranges_come_from_the_request_alone():
+    """A request's range length: 256 or 512 keys or more, whole steps of every head size's
+    kernel, at most 64 ranges a tile, and over 512 keys at most 64 of the request's tiles
+    unless a tile is one range; the same in any batch."""
+    for tiles in (1, 2, 3, 7, 32, 64, 500):
+        for ctx in (1, 511, 512, 513, 4096, 32767, 32768, 32769, 65537, 200000, 1 << 20):
+            per = pf.range_keys(tiles, ctx)
+            assert per >= 256 and per % 128 == 0 and -(-ctx // per) <= pf.MAX_RANGES
+            assert per > 256 or tiles * -(-ctx // per) <= pf.FEW_RANGES
+            assert tiles * -(-ctx // per) <= pf.MANY_RANGES or ctx <= per
+    one = (0, 40, 3000, 0)
+    other = [(40, 41, 100, 0), (41, 105, 30000, 0)]
+    alone = pf.build_tiles([one], [0], 4, "cpu").ranges.host_items
+    among = pf.build_tiles([one, *other], [0, 1, 2], 4, "cpu").ranges.host_items
+    assert (among[: len(alone), [0, 1, 2, 4]] == alone[:, [0, 1, 2, 4]]).all()
 
 
 def test_fused_range_plan_covers_every_tile_within_its_rows():
@@ -104,12 +111,12 @@ def test_fused_range_plan_covers_every_tile_within_its_rows():
         for gqa, heads, d in ((4, 8, 128), (8, 1, 128), (1, 32, 64), (4, 8, 256)):
             tiles = pf.build_tiles(prefill, list(range(len(prefill))), gqa, "cpu", tokens=pf.block_m(gqa, d))
             plan = tiles.ranges
-            items, merges = plan.items.view(-1, 4).tolist(), plan.merges.view(-1, 4).tolist()
+            items, merges = plan.items.view(-1, 5).tolist(), plan.merges.view(-1, 5).tolist()
             want = []
-            for t, (_, n, p0, ctx, _) in enumerate(tiles.tolist()):
-                per, keys = int(pf.range_keys(np.array([ctx]), d)[0]), min(p0 + n, ctx)
-                want += [(t, z, -(-keys // per), n * gqa) for z in range(-(-keys // per))]
-            assert [(i // 64, i % 64, n, r) for i, n, _, r in items] == want
+            for t, (_, n, p0, ctx, req) in enumerate(tiles.tolist()):
+                per, keys = pf.range_keys(int((tiles[:, 4] == req).sum()), ctx), min(p0 + n, ctx)
+                want += [(t, z, -(-keys // per), per, n * gqa) for z in range(-(-keys // per))]
+            assert [(i // 64, i % 64, n, per, r) for i, n, per, _, r in items] == want
             assert merges == [it for it in items if it[0] % 64 == 0 and it[1] > 1]
             for limit in (1, 1000, pf.PARTIAL_BYTES // (heads * (d + 2) * 4)):
                 groups, most = plan.groups(limit)
@@ -119,7 +126,7 @@ def test_fused_range_plan_covers_every_tile_within_its_rows():
                 for i0, n, m0, nm, row0 in g:
                     used, at = 0, row0
                     assert merges[m0 : m0 + nm] == [it for it in items[i0 : i0 + n] if it[0] % 64 == 0 and it[1] > 1]
-                    for _, ranges, first, rows in merges[m0 : m0 + nm]:
+                    for _, ranges, _, first, rows in merges[m0 : m0 + nm]:
                         assert first == at
                         at += ranges * rows
                     used = at - row0
