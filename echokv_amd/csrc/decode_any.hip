@@ -107,7 +107,7 @@ __global__ __launch_bounds__(kDecThreads, FAST && GS * NO == 1 ? 4 : 2) void dec
 
   // ---- the chain of loads: block table, header, codes ------------------------
   // As in prefill.hip: nothing loaded is looked at before the batch that needs it,
-  // and no load sits in a branch (addresses are clamped).
+  // and no load sits in a branch (addresses are clamped), but for the K statistics' mask.
   auto block_of = [&](int kp) { return FAST ? kp >> a.bs_shift : kp / L.BS; };
   auto group_of = [&](int off) { return FAST ? off >> a.kg_shift : off / L.KG; };
   auto item_key = [&](int b) { return t_begin + b * BK + 4 * row; };
@@ -148,14 +148,14 @@ __global__ __launch_bounds__(kDecThreads, FAST && GS * NO == 1 ? 4 : 2) void dec
     const uint8_t *pg, *row;  // the block's page; the item's first row (no chunk: the page)
     int rowb;                 // bytes per row (no chunk: 0)
     int bits, off;
-    bool ok;
+    bool ok;                  // the item can be read (its block and its chunk are in the layer)
   };
   auto at_of = [&](int b, const Head& x) {
     At t;
     t.off = item_off(b);
     t.bits = tier_of(x.hd().tag);
     const long rb = item_row(x, t.off, t.bits);
-    t.ok = rb >= 0;
+    t.ok = rb >= 0 && (unsigned)x.blk < (unsigned long)L.nb;
     t.pg = a.pages + page_of(x.blk) * L.stride;
     t.row = t.ok ? a.pages + rb : t.pg;
     t.rowb = t.ok ? L.H * (D / 4) * t.bits : 0;
@@ -182,8 +182,12 @@ __global__ __launch_bounds__(kDecThreads, FAST && GS * NO == 1 ? 4 : 2) void dec
 #pragma unroll
       for (int i = 0; i < 4; ++i) rk.k[n][i] = *(const uint2*)(p + i * t.rowb);
       const int se = (group_of(t.off) * L.H + h) * D + ch0(n);
-      rk.ks[n] = *(const uint4*)(t.pg + L.o_ks + 2 * se);
-      rk.km[n] = *(const uint4*)(t.pg + L.o_km + 2 * se);
+      // Lanes past the head keep the zeros they began with (selects on the loaded words: 1 %
+      // of the kernel's time more).
+      if (!past(n)) {
+        rk.ks[n] = *(const uint4*)(t.pg + L.o_ks + 2 * se);
+        rk.km[n] = *(const uint4*)(t.pg + L.o_km + 2 * se);
+      }
     }
   };
   auto load_v = [&](const At& t) {
@@ -225,6 +229,8 @@ __global__ __launch_bounds__(kDecThreads, FAST && GS * NO == 1 ? 4 : 2) void dec
   Head head1 = load_head(load_blk(wv + kDecWaves));
   int blk2 = load_blk(wv + 2 * kDecWaves);
   At at = at_of(wv, head);
+#pragma unroll
+  for (int n = 0; n < NO; ++n) rk.ks[n] = rk.km[n] = uint4{};
   load_k(head, at);
   load_v(at);
 
@@ -276,8 +282,8 @@ __global__ __launch_bounds__(kDecThreads, FAST && GS * NO == 1 ? 4 : 2) void dec
       if constexpr (FAST) {
         h2_t c[4][4];
         pairs(rk.k[n], n, at.bits, c);
-        const uint4 ks = past(n) ? uint4{} : rk.ks[n], km = past(n) ? uint4{} : rk.km[n];
-        const uint32_t sw[4] = {ks.x, ks.y, ks.z, ks.w}, mw[4] = {km.x, km.y, km.z, km.w};
+        const uint32_t sw[4] = {rk.ks[n].x, rk.ks[n].y, rk.ks[n].z, rk.ks[n].w};
+        const uint32_t mw[4] = {rk.km[n].x, rk.km[n].y, rk.km[n].z, rk.km[n].w};
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
           float x[8];
@@ -368,9 +374,9 @@ __global__ __launch_bounds__(kDecThreads, FAST && GS * NO == 1 ? 4 : 2) void dec
         pairs(rv.v[n], n, cat.bits, c);
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
-          // Keys past the split, rows without a chunk and blocks left out add zeros: their bytes
-          // are arbitrary, and a weight of 0 times an infinity is not 0.
-          const bool live = opened && cat.ok && i < n_live;
+          // Keys past the split, rows without a chunk and blocks left out (!ok) add zeros: their
+          // bytes are arbitrary, and a weight of 0 times an infinity is not 0.
+          const bool live = cat.ok && i < n_live;
           const float vs = live ? (float)u2h(rv.vs[n][i])[0] : 0.f, vm = live ? (float)u2h(rv.vm[n][i])[0] : 0.f;
           float x[8];
 #pragma unroll
