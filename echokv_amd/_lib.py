@@ -119,6 +119,12 @@ def ptr(t: torch.Tensor | None):
     return None if t is None else t.data_ptr()
 
 
+def host_i64(rows: list):
+    """Rows of integers as a C array for the length of a call."""
+    flat = [x for r in rows for x in r]
+    return (C.c_int64 * len(flat))(*flat)
+
+
 def stream() -> int:
     return torch.cuda.current_stream().cuda_stream
 

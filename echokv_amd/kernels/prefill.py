@@ -46,6 +46,7 @@ FUSED_MAX_CHUNK = 64  # the fused kernel only when every chunk is this short
 # Key ranges of the fused kernel's contexts (range_keys): a tile's most, a request's most, and
 # a request's most of 256 keys.
 MAX_RANGES, MANY_RANGES, FEW_RANGES = 64, 64, 32
+ONE_RANGE = 384  # a context of so many keys is not cut (300 keys: two ranges of 256 cost what they save)
 # Float32 partial rows of the ranges that run together; a step with more runs its tiles in
 # several launches over the same rows, each with a tail of its own: 64 chunks of 16-32 tokens
 # over 1-4K keys in ranges of 512 take 394 us at 64 MiB, 374 at 128 and 337 at 256 (a single
@@ -84,7 +85,7 @@ def range_keys(tiles: int, ctx: int) -> int:
     over 1000 keys: 28 us at 256, 47 at 512; 2 over 4096: 40, 55; but 2 requests of 2 over 8192: 86,
     74). A full batch pays for partial rows that one range per tile does without (64 chunks
     of 64 tokens over 1024 keys 209 -> 342 us; over 1-4K keys 350 -> 354)."""
-    if ctx <= 512:
+    if ctx <= ONE_RANGE:
         return 512
     per = 256 if tiles * -(-ctx // 256) <= FEW_RANGES else 512
     while 256 < per < ctx and tiles * -(-ctx // per) > MANY_RANGES:  # at most MAX_RANGES with one tile
@@ -112,21 +113,24 @@ class RangePlan:
         z = np.arange(len(t)) - np.repeat(self.n_items[:-1], n)
         items = np.stack([t * MAX_RANGES + z, n[t], per[t], self.n_rows[t], rows[t]], 1).astype(np.int32)
         self.host_items, self.host_merges = items, items[(z == 0) & (n[t] > 1)]
+        self.rows = int(self.n_rows[-1])  # partial rows per KV head
         self.items = self.merges = None
         self._groups: dict = {}
 
-    def groups(self, limit: int) -> tuple[torch.Tensor, int]:
-        """(host table [groups, 5], partial rows of the largest group): runs of tiles with at
+    def groups(self, limit: int) -> tuple[list, int]:
+        """(host rows [groups][5], partial rows of the largest group): runs of tiles with at
         most ``limit`` partial rows together (or one tile)."""
+        if self.rows <= limit:
+            return [[0, len(self.host_items), 0, len(self.host_merges), 0]], self.rows
         if limit not in self._groups:
             out, most, t, end = [], 0, 0, len(self.n_items) - 1
             while t < end:
                 u = max(t + 1, int(np.searchsorted(self.n_rows, self.n_rows[t] + limit, "right")) - 1)
-                at = [(c[t], c[u] - c[t]) for c in (self.n_items, self.n_merges, self.n_rows)]
+                at = [(int(c[t]), int(c[u] - c[t])) for c in (self.n_items, self.n_merges, self.n_rows)]
                 out.append([*at[0], *at[1], at[2][0]])
-                most = max(most, int(at[2][1]))
+                most = max(most, at[2][1])
                 t = u
-            self._groups[limit] = torch.tensor(np.array(out, np.int64)), most
+            self._groups[limit] = out, most
         return self._groups[limit]
 
 
@@ -428,12 +432,13 @@ def prefill_attention_fused(store, query: torch.Tensor, output: torch.Tensor, pr
         tiles = _upload_tiles(tiles.cpu().to(torch.int32).numpy(), gqa, tile_m, query.device)
     plan, ranges = getattr(tiles, "ranges", None), (None, None, None, 0, None, None)
     tiles = tiles.to(torch.int32).contiguous()
-    if kernels_take(L.head_size, gqa) and plan.n_merges[-1] > 0:
+    if kernels_take(L.head_size, gqa) and plan.rows > 0:
         h, d = L.num_kv_heads, L.head_size
         groups, most = plan.groups(max(1, PARTIAL_BYTES // (h * (d + 2) * 4)))
         partial = torch.empty(most * h * (d + 2), device=query.device, dtype=torch.float32)
         acc, ml = partial[: most * h * d], partial[most * h * d :]
-        ranges = (*map(_lib.ptr, (plan.items, plan.merges, groups)), groups.shape[0], _lib.ptr(acc), _lib.ptr(ml))
+        ranges = (_lib.ptr(plan.items), _lib.ptr(plan.merges), _lib.host_i64(groups), len(groups), _lib.ptr(acc),
+                  _lib.ptr(ml))
     res = _lib.residual(store.res_k)
     _lib.call(
         "echokv_prefill_split", _lib.byref(store.abi), _lib.ptr(store.pages), _lib.ptr(store.block_res),

@@ -89,6 +89,7 @@ def test_fused_key_ranges_come_from_the_request_alone():
         for ctx in (1, 511, 512, 513, 4096, 32767, 32768, 32769, 65537, 200000, 1 << 20):
             per = pf.range_keys(tiles, ctx)
             assert per >= 256 and per % 128 == 0 and -(-ctx // per) <= pf.MAX_RANGES
+            assert ctx > pf.ONE_RANGE or ctx <= per
             assert per > 256 or tiles * -(-ctx // per) <= pf.FEW_RANGES
             assert tiles * -(-ctx // per) <= pf.MANY_RANGES or ctx <= per
     one = (0, 40, 3000, 0)
@@ -119,8 +120,7 @@ def test_fused_range_plan_covers_every_tile_within_its_rows():
             assert [(i // 64, i % 64, n, per, r) for i, n, per, _, r in items] == want
             assert merges == [it for it in items if it[0] % 64 == 0 and it[1] > 1]
             for limit in (1, 1000, pf.PARTIAL_BYTES // (heads * (d + 2) * 4)):
-                groups, most = plan.groups(limit)
-                g = groups.tolist()
+                g, most = plan.groups(limit)
                 assert [sum(x[1] for x in g[:i]) for i in range(len(g) + 1)] == [x[0] for x in g] + [len(items)]
                 assert [sum(x[3] for x in g[:i]) for i in range(len(g) + 1)] == [x[2] for x in g] + [len(merges)]
                 for i0, n, m0, nm, row0 in g:
