@@ -40,8 +40,8 @@
 // than 2^8 (probabilities stay <= 256, far inside fp16).
 //
 // A split covers max(blocks_per_split, ceil(blocks / num_splits)) blocks of
-// the sequence's own length, fewer for short sequences (split_blocks), so results do not depend on the rest of the
-// batch; a second kernel merges the splits in order (log-sum-exp, log2 units).
+// the sequence's own length, fewer for short sequences (split_blocks), so results do not
+// depend on the rest of the batch; a second kernel merges the splits in order (log-sum-exp, log2 units).
 #include "items.h"
 
 namespace ek {
@@ -1293,8 +1293,7 @@ template <int CTRL, int ROWS>
 __device__ __forceinline__ int dpp_add(int x) {
   return x + __builtin_amdgcn_update_dpp(0, x, CTRL, ROWS, 0xF, false);
 }
-__device__ __forceinline__ int wave_incl_scan(int x, int lane) {
-  (void)lane;
+__device__ __forceinline__ int wave_incl_scan(int x) {
   x = dpp_add<0x111, 0xF>(x);
   x = dpp_add<0x112, 0xF>(x);
   x = dpp_add<0x114, 0xF>(x);
@@ -1326,7 +1325,7 @@ __device__ __forceinline__ int scan_chunk(const DecodeArgs& a, long s0, int lane
     const int bps = split_blocks(a.sp, nb);
     x = (((nb + bps - 1) / bps - 1) << 7) | 1;
   }
-  return wave_incl_scan(x, lane);
+  return wave_incl_scan(x);
 }
 __device__ __forceinline__ int scan_total(int incl) {
   const int t = __builtin_amdgcn_readlane(incl, 63);
