@@ -178,12 +178,13 @@ struct DenseArgs {
 // is a serial chain of tiles, and such sequences would be one or two of them however
 // idle the chip is (one 1337-token request, 64-token blocks, INT4: 72 us in two splits of
 // 1024 tokens, 45 in three). The rule looks at the sequence alone, so it also holds where the
-// batch fills the chip, and there every further split costs about 12 us of one
-// workgroup: cutting longer sequences finer too takes 128 x 2048 tokens from 129 us (1024 a
-// split) to 132 (512) or 147 (256), so they keep bps. cut4 = cut3 = min = 0: bps alone. Up to cap blocks num_splits splits of
-// the size above always suffice, which leaves the division by num out of the start-up
-// chain of every workgroup and merge wave (48 x 0.5-8K tokens at two tiers, three tier passes:
-// 161.9 -> 158.0 us; 64 x 0.5-8K at one: 115.9 -> 115.2).
+// batch fills the chip. Short sequences gain there too, their splits balance (256 x 200-1000
+// tokens: 160 -> 147 us at 64-token blocks, 251 -> 217 at 16; 256 x 900-1024 193 -> 180; 400 x
+// 500-1000 359 -> 310; 512 x 100-400 430 -> 342), longer ones would lose: 128 x 2048 tokens take
+// 129 us at 1024 a split, 132 at 512, 147 at 256, so they keep bps. cut4 = cut3 = min = 0: bps
+// alone. Up to cap blocks num_splits splits of the size above always suffice, which leaves
+// the division by num out of the start-up chain of every workgroup and merge wave (48 x
+// 0.5-8K tokens at two tiers, three tier passes: 161 -> 159 us; 64 x 0.5-8K at one: no difference).
 struct Splits {
   int num, bps, cut4, cut3, min, cap;
 };

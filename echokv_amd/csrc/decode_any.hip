@@ -7,15 +7,16 @@
 //
 // One workgroup per (sequence, KV head, split, group of query heads) in fp32 arithmetic,
 // the split schedule of the MFMA kernels (splits of max(blocks_per_split, ceil(blocks /
-// num_splits)) blocks, fewer for short sequences, so a sequence's result does not depend on its batch) and
+// num_splits)) blocks, fewer for short sequences, so a sequence's result does not depend on
+// its batch) and
 // the same workspace rows: acc [S, Hq, splits, D] unnormalized, ml (running max
 // in log2 units, sum). Keys and values go from codes to registers to products: a lane
 // holds 8 channels of its query heads and of O, a row of 16 lanes (8 up to head size
 // 64) a key's head, so a key costs its products, 4 lane sums per query head and one
 // exponential, and no LDS. 16 sequences of 0.2-4K tokens, INT4, H 8, GQA 4, D 96, V group
-// 24: 2150 us with keys staged 64 at a time over scalar loads, 63 us now; a wave's
-// batch of 16 keys takes 2 us (its vector instructions, two waves a SIMD), and a
-// split of 1024 tokens is 16 of them.
+// 24, with the merge: 2123 us with keys staged 64 at a time over scalar loads, 68 us now; a
+// wave's batch of 16 keys takes 2 us (its waves, two a SIMD, issue in half of their cycles),
+// and a split of 1024 tokens is 16 of them.
 //
 // Each token is dequantized as the reference's gather does: K codes with the
 // group's per-channel (scale, min), or the residual row for the open group; V

@@ -21,9 +21,9 @@
 // context is cut into ranges, one workgroup each; a range leaves
 // its rows' unnormalized output and (max, sum), and prefill_merge_kernel adds them.
 // A tile whose context is one range writes its rows directly. 4 chunks of 5-64
-// tokens over 0.7-8K-token INT4 contexts, H 8, D 128: 850 us in one range per pair, 61 us
-// cut into 400 (55 in this kernel, at 2 workgroups a CU bound by its vector
-// instructions: dequantization and softmax; 6 in the merge).
+// tokens over 0.7-8K-token INT4 contexts, H 8, D 128: 857 us in one range per pair, 55 us
+// cut (about 50 in this kernel, whose waves, two a SIMD, issue in 38 % of their cycles and
+// wait for loads, barriers and one another in the rest; 5 in the merge).
 //
 // A thread dequantizes one item of a step: 4 consecutive keys (one block, chunk and K
 // group) x 8 channels, so one 16-byte load each of K scale and K min serves four

@@ -763,7 +763,7 @@ __global__ __launch_bounds__(kThreads) void write_step_kernel(StepArgs s) {
 // fused kernel's fin rows of up to 64 keys leave its token rows 3 waves a SIMD), in
 // the pair's order, so no residual store is handed over and no token row looks through
 // the fin rows. 8155 rows of 3 requests (INT4, H 8, D 128, bf16, 254 fin
-// rows): 66 us fused, 14 + 14 us here (1.6 TB/s of the bytes it cannot do without).
+// rows): 63.5 us fused, 14 + 14 us here (1.6 TB/s of the bytes it cannot do without).
 // ---------------------------------------------------------------------------
 template <int DT, int TPT>
 __global__ __launch_bounds__(kThreads) void fin_rows_kernel(StepArgs s) {
