@@ -14,7 +14,7 @@
 // holds 8 channels of its query heads and of O, a row of 16 lanes (8 up to head size
 // 64) a key's head, so a key costs its products, 4 lane sums per query head and one
 // exponential, and no LDS. 16 sequences of 0.2-4K tokens, INT4, H 8, GQA 4, D 96, V group
-// 24, with the merge: 2123 us with keys staged 64 at a time over scalar loads, 68 us now; a
+// 24, with the merge: 2116 us with keys staged 64 at a time over scalar loads, 68 us now; a
 // wave's batch of 16 keys takes 2 us (its waves, two a SIMD, issue in half of their cycles),
 // and a split of 1024 tokens is 16 of them.
 //

@@ -512,7 +512,7 @@ def test_layouts_outside_the_mfma_kernels(device, d, bs, kg, vg, h, gqa, bits):
     (64, 32, 8, 32, 3, 7, torch.float32),     # two workgroups of query heads
     (96, 64, 32, 24, 4, 1, torch.float16),    # one query head
     (160, 16, 16, 32, 2, 3, torch.bfloat16),  # two items a lane, the second ones partly past the head
-    (36, 16, 16, 12, 2, 5, torch.float32),    # half an octet: element by element
+    (36, 16, 16, 12, 2, 5, torch.float32),    # half an octet: runs of four channels
     (128, 32, 4, 64, 2, 4, torch.float16)])   # a K group is one item
 @pytest.mark.parametrize("bits", [8, 4, 2])
 def test_fp32_decode_items_at_their_edges(device, d, bs, kg, vg, h, gqa, dt, bits):
@@ -925,6 +925,12 @@ def test_decode_bits_do_not_depend_on_whose_workspace_it_is(device):
         assert torch.equal(dec.decode_attention(store, q, table_d, lens_d, d ** -0.5, workspace=ws), own)
     with pytest.raises(ValueError, match="fewer than"):
         dec.decode_attention(store, q, table_d, lens_d, d ** -0.5, workspace=pair(len(lens)))
+    # More sequences than 64 MiB hold four splits of: the static call keeps the splits the lengths need.
+    s = dec.STATIC_BYTES // (4 * gqa * h * (d + 2) * 4) + 1
+    many = (q[:1].expand(s, -1, -1).contiguous(), table_d[1:2, :3].expand(s, -1).contiguous(),
+            torch.full((s,), 130, device=device))
+    got = dec.decode_attention(store, *many, d ** -0.5, workspace="static")
+    check("static workspace, many sequences", got[-1], dec.decode_attention(store, *many, d ** -0.5)[-1].cpu().numpy())
 
 
 def test_fused_prefill_with_a_scale_that_is_not_a_number(device):
